@@ -28,12 +28,12 @@ METRIC = "Poisson apply s/tree + GFLOP/s (order 7, \u03b5=1e-6), chosen vs plain
 
 
 def band_kernel(precision, order=7):
-    """Name of the band kernel that runs: at order 7 the FP64 and FP32 sweeps
-    use the wave-owned-row kernel (unless the tile layout is selected), every
-    other case the tile-shared one."""
+    """Family of the band kernel that runs: the one-wave-per-item kernels for
+    FP64 at every order and FP32 at order 7 (unless the tile layout is selected
+    there), the tile-shared one otherwise."""
     import mrcpp_amd as mr
-    if order == 7 and precision in ("fp64", "fp32") and mr.band_layout() != "tiles":
-        return "k_band_rows"
+    if (precision == "fp64" and order != 7) or (order == 7 and precision in ("fp64", "fp32") and mr.band_layout() != "tiles"):
+        return "k_band_waves"
     return "k_band_mfma"
 COPY_PROBE_BYTES = 256 << 20
 

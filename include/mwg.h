@@ -360,12 +360,12 @@ mwg_status mwg_hash_update_multi(const mwg_hash_table *tables, int ntables, cons
 mwg_status mwg_band_apply(const mwg_level *lvl, const mwg_pairs *pairs, int npairs, int precision);
 
 /* Work distribution of the matrix-core band kernel at order 7 (kp1 = 8) for
- * MWG_PREC_FP64 and MWG_PREC_FP32.  MWG_BAND_ROWS: each wave of a workgroup
- * owns 16 rows of every sweep, so only the x -> y step crosses waves (one
- * workgroup barrier per group) and the z sweep is shared evenly whatever the
- * group's gt mask.  MWG_BAND_TILES: the tiles of each sweep are shared out
- * over the waves (two barriers per group), the layout of every other order
- * and precision.  MWG_BAND_AUTO (the default) is MWG_BAND_ROWS where it
+ * MWG_PREC_FP64 and MWG_PREC_FP32.  MWG_BAND_ROWS: each wave runs all three
+ * sweeps of a work unit for its own output columns (one gx, four j0), with no
+ * workgroup barrier; the FP64 sweeps of the other orders always do.
+ * MWG_BAND_TILES: the tiles of each sweep are shared out over the waves (two
+ * barriers per group), the layout of the other orders' FP32 and of BF16X3.
+ * MWG_BAND_AUTO (the default) is MWG_BAND_ROWS where it
  * applies.  The layouts give bit-identical results.  Process-wide; no
  * reference counterpart. */
 enum { MWG_BAND_AUTO = 0, MWG_BAND_TILES = 1, MWG_BAND_ROWS = 2 };
@@ -374,8 +374,8 @@ int mwg_band_layout(void);
 
 /* Launch parameters of the band sum, process-wide: each work unit holds at
  * least unit_groups groups of an output node (default 32; 8..1024), and the
- * persistent band kernels run at most workgroups_per_cu workgroups per
- * compute unit (0, the default: as many as fit).  Results depend on
+ * persistent band kernels run at most workgroups_per_cu workgroups (of four
+ * waves) per compute unit (0, the default: as many as fit).  Results depend on
  * unit_groups only through the order in which a node's partial sums are
  * added (last bits); the defaults are what the parity tests hold.  No
  * reference counterpart (the launch shape of calcNodeVector's work). */

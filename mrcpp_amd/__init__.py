@@ -522,8 +522,8 @@ BAND_LAYOUTS = {"auto": 0, "tiles": 1, "rows": 2}
 
 def set_band_layout(name):
     """Work distribution of the order-7 FP64/FP32 band kernel (process-wide):
-    'rows' (each wave owns 16 rows of every sweep, one workgroup barrier per
-    group), 'tiles' (sweep tiles shared out over the waves, two barriers per
+    'rows' (each wave runs all sweeps for its own output columns, no workgroup
+    barrier), 'tiles' (sweep tiles shared out over the waves, two barriers per
     group) or 'auto' (the default: 'rows').  Results are bit-identical."""
     if name not in BAND_LAYOUTS:
         raise ValueError("band layout must be one of %s" % sorted(BAND_LAYOUTS))

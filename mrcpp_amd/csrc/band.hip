@@ -13,13 +13,14 @@
 //     output node are cut into work units of at most G consecutive groups
 //     (G grows with the level so the partial results fit a fixed budget), and
 //     the group codes are copied into level order.
-//  3. k_band_mfma (matrix cores) or k_band_units (vector ALUs): persistent
-//     workgroups take units from an atomic counter; a unit accumulates its
-//     groups' 3-sweep tensor products in registers and writes one 8-block
-//     result, the node's first unit straight into the output coefficients,
-//     later units into partial slots.
-//  4. k_reduce_units: per output node and chunk of coefficients, the partial
-//     slots are added in unit order; k_level_norms computes the component
+//  3. k_band_waves* (band_waves.h: FP64, and FP32 at order 7), k_band_mfma (the
+//     other matrix-core cases) or k_band_units (vector ALUs): persistent
+//     workgroups take units in turn or from an atomic counter; a unit
+//     accumulates its groups' 3-sweep tensor products in registers and writes
+//     one 8-block result, into partial slots or, as a node's only unit (with
+//     the latter two kernels also as its first), the output coefficients.
+//  4. k_reduce_waves / k_reduce_units: per output node and chunk of
+//     coefficients, the partial slots are added in unit order; k_level_norms computes the component
 //     norms (MWNode::calcNorms, src/trees/MWNode.cpp:609-655).
 // Every summation order is fixed by the pair and group order, so results do
 // not depend on scheduling.
@@ -248,9 +249,11 @@ __device__ inline int units_group_size(int gmin, int total, int slots, int T) {
     return max(G, (T + kMaxUnitsPerNode - 1) / kMaxUnitsPerNode);
 }
 
-// Units per output node, packed with a nonzero flag so one scan yields both
-// the first unit and the first partial slot of every node.
-__global__ __launch_bounds__(256) void k_unit_count(int L, mwg_pairs pr, int npairs, const int *gstart, int gmin, int slots, long long *packed, int *counter,
+// Units per output node, packed with a flag so one scan yields both the first
+// unit and the first partial slot of every node.  With all_slots (the wave
+// kernels) a node of several units has a slot for each, else for each but the
+// first, which writes the node itself; the flag marks the units without one.
+__global__ __launch_bounds__(256) void k_unit_count(int L, mwg_pairs pr, int npairs, const int *gstart, int gmin, int slots, bool all_slots, long long *packed, int *counter,
                                                     const mwg_segment *segs, const int *node_seg, const int *papp, const double *pmg, double *g_margin) {
     const int g = blockIdx.x * 256 + threadIdx.x;
     if (g == 0) *counter = 0;
@@ -290,23 +293,58 @@ __global__ __launch_bounds__(256) void k_unit_count(int L, mwg_pairs pr, int npa
     const int T = gstart[gf + np] - gstart[gf];
     const int G = units_group_size(gmin, gstart[npairs], slots, T);
     const int nu = (T + G - 1) / G;
-    packed[g] = (long long)nu + ((long long)(nu > 0) << 32);
+    packed[g] = (long long)nu + ((long long)(all_slots ? nu == 1 : nu > 0) << 32);
 }
 
 __device__ inline int unit_first(long long v) { return (int)(v & 0xffffffffll); }
-__device__ inline int nonzero_before(long long v) { return (int)(v >> 32); }
+__device__ inline int flagged_before(long long v) { return (int)(v >> 32); }
 
-// One wave per pair: the descriptors {pair, first group in the pair, groups,
-// partial slot or -1} of the units that start inside the pair and, when grec
-// is given, the pair's group codes in level order (gstart numbering) with the
-// pair index.
+// What a wave kernel reads of a unit and of a group, written here so that it
+// needs no chain of lookups.  Unit (three int4): operand table, band
+// coefficient pool and result address (64 bits each), first group, number of
+// groups, whether the result is the output node itself.  Group (one int4, level
+// order): x block | gt mask << 24, y block | f bits 32-42 << 21, z block | f
+// bits 43-53 << 21, f bits 0-31; a block is 2 (b40 + dl) + f bit of its
+// direction (21 bits), f the offset of the group's band block.
+struct WaveRecords {
+    int4 *unit, *group; // null: not a wave kernel
+    const mwg_segment *segs;
+    const int *node_seg;
+    const long long *g_off;
+    const int4 *pdl;
+    const long long *pfo;
+    double *partial;
+    int prec, n3;
+};
+constexpr int kUnitInts = 12;
+
+// One wave per pair: the descriptors of the units that start inside the pair
+// ({pair, first group in the pair, groups, partial slot or -1}, or a wave
+// kernel's) and, for the matrix-core kernels, the pair's groups in level order
+// (gstart numbering; grec: code and pair index, or a wave kernel's records).
 __global__ __launch_bounds__(64) void k_unit_write(int npairs, mwg_pairs pr, const int *gstart, const long long *uscan, int gmin, int slots, int4 *units,
-                                                   const unsigned *codes, int stride, int2 *grec) {
+                                                   const unsigned *codes, int stride, int2 *grec, WaveRecords wr) {
     const int p = blockIdx.x;
     const int base = gstart[p], cnt = gstart[p + 1] - base;
     if (cnt == 0) return;
-    if (grec)
+    if (wr.group) {
+        const int4 d = wr.pdl[p];
+        const long long fo = wr.pfo[p];
+        for (int k = threadIdx.x; k < cnt; k += 64) {
+            const unsigned code = codes[(size_t)p * stride + k];
+            const int ft = code_ft(code), b = code_block(code);
+            const long long f = fo + (long long)ft * wr.n3;
+            const unsigned fh = (unsigned)(f >> 32);
+            int4 r;
+            r.x = (int)((unsigned)((b + d.x) * 2 + (ft & 1)) | (code_mask(code) << 24));
+            r.y = (int)((unsigned)((b + d.y) * 2 + ((ft >> 1) & 1)) | (fh << 21));
+            r.z = (int)((unsigned)((b + d.z) * 2 + ((ft >> 2) & 1)) | ((fh >> 11) << 21));
+            r.w = (int)(unsigned)f;
+            wr.group[base + k] = r;
+        }
+    } else if (grec) {
         for (int k = threadIdx.x; k < cnt; k += 64) grec[base + k] = make_int2((int)codes[(size_t)p * stride + k], p);
+    }
     if (threadIdx.x != 0) return;
     const int g = pr.pair_g[p];
     const int gf = pr.g_first[g], np = pr.g_npairs[g];
@@ -316,9 +354,23 @@ __global__ __launch_bounds__(64) void k_unit_write(int npairs, mwg_pairs pr, con
     const int a = base - B, e = a + cnt;
     const long long v = uscan[g];
     const int Ug = unit_first(v);
-    const int Sg = Ug - nonzero_before(v);
-    for (int j = (a + G - 1) / G; j * G < e; j++)
-        units[Ug + j] = make_int4(p, j * G - a, min(G, T - j * G), j == 0 ? -1 : Sg + j - 1);
+    const int Sg = Ug - flagged_before(v);
+    if (!wr.unit) {
+        for (int j = (a + G - 1) / G; j * G < e; j++) units[Ug + j] = make_int4(p, j * G - a, min(G, T - j * G), j == 0 ? -1 : Sg + j - 1);
+        return;
+    }
+    const mwg_segment &S = wr.segs[wr.node_seg[g]];
+    double *node = S.g_coef + wr.g_off[g];
+    auto lo = [](const void *q) { return (int)(unsigned)reinterpret_cast<unsigned long long>(q); };
+    auto hi = [](const void *q) { return (int)(unsigned)(reinterpret_cast<unsigned long long>(q) >> 32); };
+    for (int j = (a + G - 1) / G; j * G < e; j++) {
+        const bool direct = T <= G;
+        const double *out = direct ? node : wr.partial + (size_t)(Sg + j) * 8 * wr.n3;
+        int4 *u = wr.unit + (kUnitInts / 4) * (size_t)(Ug + j);
+        u[0] = make_int4(lo(S.op.frag[wr.prec]), hi(S.op.frag[wr.prec]), lo(S.f.coef), hi(S.f.coef));
+        u[1] = make_int4(lo(out), hi(out), B + j * G, min(G, T - j * G));
+        u[2] = make_int4(direct ? 1 : 0, 0, 0, 0);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -923,238 +975,15 @@ __global__ __launch_bounds__(256, N1 == 10 ? 2 : 1) void k_band_mfma(const mwg_s
     }
 }
 
-// ---------------------------------------------------------------------------
-// 3c. order 7 (N1 = 8) on the matrix cores with wave-owned rows (FP64, FP32).
-//
-// The same sweeps and instructions as k_band_mfma<8, PREC>, distributed so
-// that only the x -> y step crosses waves.  Wave w computes the x sweep rows
-// i1 + N1 i2 with i2 in {2w, 2w+1} (it writes and reads its own F rows), and
-// the y and z sweeps for the output rows with j0 in {2w, 2w+1}: the y sweep
-// reads T1 rows written by every wave (one barrier per group; T1 is kept
-// twice, by group parity, so the next group's x sweep does not wait for the
-// slowest wave's y sweep) and writes T2 rows only this wave reads; the z
-// sweep runs every needed (gx, gy) block, so the four waves do equal work
-// whatever the gt mask.  Every output element goes through the same products
-// in the same order as in k_band_mfma: the results are bit-identical.
-//
-// LDS layouts (element offsets; conflict-free for these access patterns:
-// each 32-lane half of an access touches distinct banks, and for FP64 each
-// 16-lane quarter too):
-//   F[kk = i0][m = i1 + N1 i2], T1[gx][kk = i1][j0 + N1 i2],
-//   T2 (per wave) [b = 2 gx + gy][kk = i2][r = j1 + N1 (j0 - 2w)].
-// ---------------------------------------------------------------------------
-template <int PREC> struct RowGeom;
-template <> struct RowGeom<MWG_PREC_FP64> {
-    static constexpr int F = 512, T1B = 520, T1 = 2 * T1B, T2W = 512;
-    __device__ static inline int atF(int kk, int m) { return kk * 64 + (m ^ (2 * kk) ^ (16 * (kk & 1))); }
-    __device__ static inline int atT1(int gx, int kk, int j0, int i2) { return gx * T1B + kk * 64 + (((j0 + 8 * i2) ^ (2 * (i2 >> 1))) ^ (16 * (kk & 1))); }
-    __device__ static inline int atT2(int b, int kk, int r) {
-        const int gy = b & 1;
-        return b * 128 + ((kk * 16 + (r ^ (8 * gy))) ^ (16 * gy));
-    }
-};
-template <> struct RowGeom<MWG_PREC_FP32> {
-    static constexpr int F = 512, T1B = 552, T1 = 2 * T1B, T2W = 576;
-    __device__ static inline int atF(int kk, int m) { return kk * 64 + (m ^ (16 * (kk & 1)) ^ (4 * (kk >> 1))); }
-    __device__ static inline int atT1(int gx, int kk, int j0, int i2) { return gx * T1B + kk * 68 + ((j0 + 8 * i2) ^ (2 * (i2 >> 2))); }
-    __device__ static inline int atT2(int b, int kk, int r) { return b * 144 + kk * 16 + (r ^ (8 * ((kk >> 1) & 1))); }
-};
+} // namespace
 
-// FP32: at least 5 waves per SIMD (the registers allow 4 otherwise; a few
-// spilled bytes cost less than the latency the fifth wave hides).
-template <int PREC>
-__global__ __launch_bounds__(256, PREC == MWG_PREC_FP32 ? 5 : 1) void k_band_rows(const mwg_segment *segs, const int *node_seg, const long long *g_off, mwg_pairs pr, const int2 *grec,
-                                                   const int4 *pdl, const long long *pfo, const int *gstart, const int4 *units,
-                                                   const long long *uscan, int L, double *partial, int *counter) {
-    constexpr int N1 = 8, N3 = 512, KSTEPS = 2;
-    constexpr int FRAG = KSTEPS * 64; // operand elements per (matrix block, f bit)
-    using R = RowGeom<PREC>;
-    using LT = typename BandTypes<PREC>::L;
-    using BT = typename BandTypes<PREC>::B;
-    using MM = typename BandTypes<PREC>::MM;
-    __shared__ __align__(16) LT sF[R::F];
-    __shared__ __align__(16) LT sT1[2 * R::T1];
-    __shared__ __align__(16) LT sT2[4 * R::T2W];
-    __shared__ int s_unit;
+} // namespace mwgdev
 
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int li = lane & 15, lq = lane >> 4;
-    const auto useg = ro(segs);
-    const auto unode = ro(node_seg);
-    const auto ud4 = ro(reinterpret_cast<const int *>(units));
-    const int total = unit_first(ro(uscan)[L]);
-    LT *const myT2 = sT2 + w * R::T2W;
+#include "band_waves.h"
 
-    for (int i = tid; i < R::F; i += 256) sF[i] = LT(0);
-    for (int i = tid; i < 2 * R::T1; i += 256) sT1[i] = LT(0);
-    for (int i = tid; i < 4 * R::T2W; i += 256) sT2[i] = LT(0);
+namespace mwgdev {
 
-    // this wave's F rows: band block elements 128 w + lane + 64 k
-    auto write_f = [&](const double (&v)[2]) {
-#pragma unroll
-        for (int k = 0; k < 2; k++) sF[R::atF(lane & 7, 16 * w + 8 * k + (lane >> 3))] = (LT)v[k];
-    };
-
-    for (int u; (u = take_unit(counter, &s_unit, total)) >= 0;) {
-        // unit: groups [gi0, gi0 + ng) of one output node, contiguous in level order
-        const int p0 = ud4[4 * (size_t)u], ng = ud4[4 * (size_t)u + 2], slot = ud4[4 * (size_t)u + 3];
-        const int gi0 = ro(gstart)[p0] + ud4[4 * (size_t)u + 1];
-        const int g = ro(pr.pair_g)[p0];
-        const_as4<mwg_segment> &SG = useg[unode[g]];
-        const BT *frag = static_cast<const BT *>(SG.op.frag[PREC]);
-        const double *coef = SG.f.coef;
-        double *dst = slot < 0 ? SG.g_coef + ro(g_off)[g] : partial + (size_t)slot * 8 * N3;
-        dvec4 acc[4]; // z sweep result of block b = 2 gx + gy, rows j1 + N1 (j0 - 2w), columns gz, j2
-#pragma unroll
-        for (int b = 0; b < 4; b++) acc[b] = dvec4{0.0, 0.0, 0.0, 0.0};
-
-        // group records, 64 to a chunk, lane j holding group 64 c + j (as in k_band_mfma)
-        struct Chunk {
-            int code, d0, d1, d2, flo, fhi;
-        };
-        auto load_chunk = [&](int c, Chunk &ch) {
-            const int i = 64 * c + lane;
-            if (i < ng) {
-                const int2 r = grec[gi0 + i];
-                const int4 d = pdl[r.y];
-                const long long fo = pfo[r.y];
-                ch = Chunk{r.x, d.x, d.y, d.z, (int)(unsigned)(fo & 0xffffffffll), (int)(fo >> 32)};
-            }
-        };
-        auto take = [&](const Chunk &ch, int i, Group &q) {
-            const int j = i & 63;
-            const unsigned code = (unsigned)__builtin_amdgcn_readlane(ch.code, j);
-            q.b40 = code_block(code);
-            q.ft = code_ft(code);
-            q.mask = code_mask(code);
-            q.fresh_f = code_fresh(code);
-            q.dl[0] = __builtin_amdgcn_readlane(ch.d0, j);
-            q.dl[1] = __builtin_amdgcn_readlane(ch.d1, j);
-            q.dl[2] = __builtin_amdgcn_readlane(ch.d2, j);
-            const long long fo = ((long long)__builtin_amdgcn_readlane(ch.fhi, j) << 32) | (unsigned)__builtin_amdgcn_readlane(ch.flo, j);
-            q.fsrc = coef + fo + (long long)q.ft * N3;
-        };
-        using Frags = BT[KSTEPS];
-        auto fetch = [&](const Group &q, Frags &fx, Frags &fy, Frags &fz) {
-#pragma unroll
-            for (int ks = 0; ks < KSTEPS; ks++) {
-                const int o = ks * 64 + lane;
-                fx[ks] = frag[(size_t)((q.b40 + q.dl[0]) * 2 + (q.ft & 1)) * FRAG + o];
-                fy[ks] = frag[(size_t)((q.b40 + q.dl[1]) * 2 + ((q.ft >> 1) & 1)) * FRAG + o];
-                fz[ks] = frag[(size_t)((q.b40 + q.dl[2]) * 2 + ((q.ft >> 2) & 1)) * FRAG + o];
-            }
-        };
-
-        Chunk ca{}, cb{};
-        load_chunk(0, ca);
-        if (ng > 64) load_chunk(1, cb);
-        Group ga, gb;
-        Frags ax, ay, az, bx, by, bz;
-        double fpre[2];
-        take(ca, 0, ga);
-        fetch(ga, ax, ay, az);
-        {
-            double v[2];
-#pragma unroll
-            for (int k = 0; k < 2; k++) v[k] = ga.fsrc[128 * w + lane + 64 * k];
-            write_f(v);
-        }
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        auto step = [&](int i, Group &cur, Frags &fx, Frags &fy, Frags &fz, Group &nq, Frags &nfx, Frags &nfy, Frags &nfz) -> bool {
-#pragma unroll
-            for (int ks = 0; ks < KSTEPS; ks++) {
-                settled(fx[ks]);
-                settled(fy[ks]);
-                settled(fz[ks]);
-            }
-            const bool have_next = i + 1 < ng;
-            if (have_next && ((i + 1) & 63) == 0) take(cb, i + 1, nq);
-            else take(ca, have_next ? i + 1 : i, nq);
-            const bool next_f = have_next && nq.fresh_f;
-#pragma unroll
-            for (int k = 0; k < 2; k++) fpre[k] = nq.fsrc[128 * w + lane + 64 * k];
-            fetch(nq, nfx, nfy, nfz);
-            const unsigned gm = cur.mask;
-            unsigned xneed, yneed;
-            sweep_needs(gm, xneed, yneed);
-            LT *const t1 = sT1 + (i & 1) * R::T1;
-            // x sweep, rows m = i1 + N1 i2 of this wave: T1[gx][i1][j0 + N1 i2] = sum_i0 F[i0][m] Ox_gx(i0, j0)
-            {
-                typename MM::C c = {};
-#pragma unroll
-                for (int ks = 0; ks < KSTEPS; ks++) c = MM::mma(sF[R::atF(4 * ks + lq, 16 * w + li)], fx[ks], c);
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const int rho = MM::row(lane, r);
-                    t1[R::atT1(li >> 3, rho & 7, li & 7, 2 * w + (rho >> 3))] = c[r];
-                }
-            }
-            __syncthreads();
-            // y sweep, rows (j0 = 2w + (row & 1), i2 = row >> 1):
-            // T2[gx][gy][i2][j1 + N1 (j0 - 2w)] = sum_i1 T1[gx][i1][j0 + N1 i2] Oy_gy(i1, j1)
-#pragma unroll
-            for (int gx = 0; gx < 2; gx++) {
-                if (!(xneed >> gx & 1)) continue;
-                typename MM::C c = {};
-#pragma unroll
-                for (int ks = 0; ks < KSTEPS; ks++) c = MM::mma(t1[R::atT1(gx, 4 * ks + lq, 2 * w + (li & 1), li >> 1)], fy[ks], c);
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const int rho = MM::row(lane, r);
-                    myT2[R::atT2(2 * gx + (li >> 3), rho >> 1, (li & 7) + 8 * (rho & 1))] = c[r];
-                }
-            }
-            // T2 and F rows pass between lanes of this wave only: the wave's LDS
-            // accesses complete in issue order, so a compiler fence suffices
-            __atomic_signal_fence(__ATOMIC_SEQ_CST);
-            // z sweep of every needed (gx, gy), rows j1 + N1 (j0 - 2w):
-            // G[gt][j0 + N1 j1 + N2 j2] += sum_i2 T2[gx][gy][i2][.] Oz_gz(i2, j2), columns of a gz outside the mask zeroed
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const int gx = b >> 1, gy = b & 1;
-                if (!(yneed >> (gx + 2 * gy) & 1)) continue;
-                const bool keep = (gm >> (gx + 2 * gy + 4 * (li >> 3))) & 1;
-                BT zb[KSTEPS];
-#pragma unroll
-                for (int ks = 0; ks < KSTEPS; ks++) zb[ks] = keep ? fz[ks] : BT{};
-                if constexpr (PREC == MWG_PREC_FP64) {
-#pragma unroll
-                    for (int ks = 0; ks < KSTEPS; ks++) acc[b] = MM::mma(myT2[R::atT2(b, 4 * ks + lq, li)], zb[ks], acc[b]);
-                } else {
-                    typename MM::C c = {};
-#pragma unroll
-                    for (int ks = 0; ks < KSTEPS; ks++) c = MM::mma(myT2[R::atT2(b, 4 * ks + lq, li)], zb[ks], c);
-#pragma unroll
-                    for (int r = 0; r < 4; r++) acc[b][r] += (double)c[r];
-                }
-            }
-            __atomic_signal_fence(__ATOMIC_SEQ_CST);
-            // the next band block into this wave's F rows (its x sweep above has read them)
-            if (next_f) write_f(fpre);
-            __atomic_signal_fence(__ATOMIC_SEQ_CST);
-            if (have_next && ((i + 1) & 63) == 0) {
-                ca = cb;
-                if (i + 1 + 64 < ng) load_chunk((i + 1) / 64 + 1, cb);
-            }
-            return have_next;
-        };
-        for (int i = 0;; i += 2) {
-            if (!step(i, ga, ax, ay, az, gb, bx, by, bz)) break;
-            if (!step(i + 1, gb, bx, by, bz, ga, ax, ay, az)) break;
-        }
-        // blocks gt = gx + 2 gy + 4 gz, output rows j0 in {2w, 2w + 1}
-#pragma unroll
-        for (int b = 0; b < 4; b++) {
-            const int gx = b >> 1, gy = b & 1;
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int rho = MM::row(lane, r);
-                const int j1 = rho & 7, j0 = 2 * w + (rho >> 3), gz = li >> 3, j2 = li & 7;
-                dst[(gx + 2 * gy + 4 * gz) * N3 + j0 + N1 * j1 + 64 * j2] = acc[b][r];
-            }
-        }
-    }
-}
+namespace {
 
 // Operand table of one precision from the FP64 operator matrices.  Element
 // (matrix block b4, f bit, column tile nt, step ks, lane) of P[k][n] =
@@ -1229,7 +1058,7 @@ __global__ __launch_bounds__(256) void k_reduce_units(const mwg_segment *segs, c
         dst[o] = 0.0;
         return;
     }
-    const int Sg = Ug - nonzero_before(v);
+    const int Sg = Ug - flagged_before(v);
     double acc = dst[o];
     const double *src = partial + (size_t)Sg * 8 * N3 + o;
     // slots added in unit order; their loads issued 8 at a time
@@ -1294,21 +1123,40 @@ template <int N1, int PREC> int mfma_grid() {
     static const int grid = resident_grid(k_band_mfma<N1, PREC>, 256);
     return capped_grid(grid);
 }
-template <int PREC> int rows_grid() {
-    static const int grid = resident_grid(k_band_rows<PREC>, 256);
-    return capped_grid(grid);
-}
 int g_band_layout = MWG_BAND_AUTO;
+// Whether a wave kernel runs: FP64 at every order, FP32 at order 7 (the other
+// orders' FP32 and BF16X3 sweeps keep the tile-shared kernel, as order 7 does
+// when that layout is selected).
+bool wave_kernel(int n1, int prec) {
+    if (prec == MWG_PREC_FP64) return n1 != 8 || g_band_layout != MWG_BAND_TILES;
+    return prec == MWG_PREC_FP32 && n1 == 8 && g_band_layout != MWG_BAND_TILES;
+}
+template <int N1, int PREC> void (*wave_kernel_of())(WaveArgs) {
+    if constexpr (N1 != 8) return k_band_waves<N1>;
+    else if constexpr (PREC == MWG_PREC_FP64) return k_band_waves8;
+    else return k_band_waves8f;
+}
+// Threads of a wave kernel's workgroup: the four items of a unit at order 7,
+// one item otherwise.  The grid is then a multiple of 8 units' items (WaveTurn);
+// the cap counts four waves as a workgroup.
+template <int N1> constexpr int wave_threads() { return N1 == 8 ? 256 : 64; }
+template <int N1, int PREC> int wave_grid() {
+    static const int resident = resident_grid(wave_kernel_of<N1, PREC>(), wave_threads<N1>());
+    if constexpr (N1 == 8) return capped_grid(resident);
+    constexpr int unit = 8 * WaveShape<N1>::ITEMS;
+    const int grid = g_band_wg_per_cu > 0 ? std::min(resident, 4 * g_band_wg_per_cu * device_cus()) : resident;
+    return std::max(1, grid / unit) * unit;
+}
 template <int N1, int PREC>
 void launch_mfma(const mwg_level *lvl, const LevelDevice &dev, const mwg_pairs *pr, BandWork &w, int stride) {
-    if constexpr (N1 == 8 && (PREC == MWG_PREC_FP64 || PREC == MWG_PREC_FP32)) {
-        if (g_band_layout != MWG_BAND_TILES) {
-            hipLaunchKernelGGL((k_band_rows<PREC>), dim3(rows_grid<PREC>()), dim3(256), 0, 0, dev.segs, dev.node_seg, lvl->g_off, *pr,
-                               w.grec.as<int2>(), w.pdl.as<int4>(), w.pfo.as<long long>(), w.gstart.as<int>(), w.units.as<int4>(),
-                               w.uscan.as<long long>(), lvl->count, w.partial.as<double>(), w.counter.as<int>());
+    if constexpr (PREC == MWG_PREC_FP64 || (PREC == MWG_PREC_FP32 && N1 == 8)) {
+        if (wave_kernel(N1, PREC)) {
+            const WaveArgs a{w.grec.as<int4>(), w.units.as<int>(), w.uscan.as<long long>(), lvl->count};
+            hipLaunchKernelGGL((wave_kernel_of<N1, PREC>()), dim3(wave_grid<N1, PREC>()), dim3(wave_threads<N1>()), 0, 0, a);
             return;
         }
     }
+    if constexpr (PREC != MWG_PREC_FP64 || N1 == 8)
     hipLaunchKernelGGL((k_band_mfma<N1, PREC>), dim3(mfma_grid<N1, PREC>()), dim3(256), 0, 0, dev.segs, dev.node_seg, lvl->g_off, *pr,
                        w.grec.as<int2>(), w.pdl.as<int4>(), w.pfo.as<long long>(), w.gstart.as<int>(), w.units.as<int4>(),
                        w.uscan.as<long long>(), lvl->count, w.partial.as<double>(), w.counter.as<int>());
@@ -1337,11 +1185,14 @@ template <int N1> struct BandL {
         if (w.codes.ensure(sizeof(unsigned) * (size_t)npairs * stride) != MWG_OK) return MWG_ERR_NOMEM;
         if (w.gstart.ensure(sizeof(int) * ((size_t)npairs + 1)) != MWG_OK) return MWG_ERR_NOMEM;
         if (w.uscan.ensure(sizeof(long long) * ((size_t)L + 1)) != MWG_OK) return MWG_ERR_NOMEM;
-        if (w.units.ensure(sizeof(int4) * ((size_t)slots + L)) != MWG_OK) return MWG_ERR_NOMEM;
-        if (w.partial.ensure(slot_bytes * (size_t)slots) != MWG_OK) return MWG_ERR_NOMEM;
+        const bool waves = wave_kernel(N1, precision);
+        if (w.units.ensure((waves ? sizeof(int) * kUnitInts : sizeof(int4)) * ((size_t)slots + L)) != MWG_OK) return MWG_ERR_NOMEM;
+        // with all_slots a node of several units (more than one per slot's
+        // share of groups, so at most `slots` of them) takes one more
+        if (w.partial.ensure(slot_bytes * ((size_t)slots + (waves ? std::min(slots, L) : 0))) != MWG_OK) return MWG_ERR_NOMEM;
         if (w.counter.ensure(sizeof(int)) != MWG_OK) return MWG_ERR_NOMEM;
         const bool mfma = precision != kPrecValuBand;
-        if (mfma && w.grec.ensure(sizeof(int2) * (size_t)npairs * stride) != MWG_OK) return MWG_ERR_NOMEM;
+        if (mfma && w.grec.ensure((waves ? sizeof(int4) : sizeof(int2)) * (size_t)npairs * stride) != MWG_OK) return MWG_ERR_NOMEM;
         if (w.pdl.ensure(sizeof(int4) * (size_t)npairs) != MWG_OK) return MWG_ERR_NOMEM;
         if (w.pfo.ensure(sizeof(long long) * (size_t)npairs) != MWG_OK) return MWG_ERR_NOMEM;
         if (w.papp.ensure(sizeof(int) * (size_t)npairs) != MWG_OK) return MWG_ERR_NOMEM;
@@ -1353,6 +1204,8 @@ template <int N1> struct BandL {
         }
         int *gstart = w.gstart.as<int>();
         long long *uscan = w.uscan.as<long long>();
+        const WaveRecords wr{waves ? w.units.as<int4>() : nullptr, waves ? w.grec.as<int4>() : nullptr, dev.segs, dev.node_seg, lvl->g_off,
+                             w.pdl.as<int4>(), w.pfo.as<long long>(), w.partial.as<double>(), precision, N3};
         {
             ProfileScope prof_(MWG_KERNEL_GROUPS);
             hipLaunchKernelGGL(k_group_screen, dim3(npairs), dim3(64 * kScreenWaves), 0, 0, dev.segs, dev.node_seg, lvl->l, lvl->node_thr, *pr,
@@ -1360,13 +1213,13 @@ template <int N1> struct BandL {
             MWG_LAUNCHED();
             mwg_status s = scan_exclusive(gstart, gstart, npairs);
             if (s != MWG_OK) return s;
-            hipLaunchKernelGGL(k_unit_count, dim3((L + 255) / 256), dim3(256), 0, 0, L, *pr, npairs, gstart, g_unit_groups, slots, uscan, w.counter.as<int>(),
+            hipLaunchKernelGGL(k_unit_count, dim3((L + 255) / 256), dim3(256), 0, 0, L, *pr, npairs, gstart, g_unit_groups, slots, waves, uscan, w.counter.as<int>(),
                                dev.segs, dev.node_seg, w.papp.as<int>(), mg.pair, lvl->g_margin);
             MWG_LAUNCHED();
             s = scan_exclusive(uscan, uscan, L);
             if (s != MWG_OK) return s;
             hipLaunchKernelGGL(k_unit_write, dim3(npairs), dim3(64), 0, 0, npairs, *pr, gstart, uscan, g_unit_groups, slots, w.units.as<int4>(), w.codes.as<unsigned>(),
-                               stride, mfma ? w.grec.as<int2>() : nullptr);
+                               stride, mfma ? w.grec.as<int2>() : nullptr, wr);
             MWG_LAUNCHED();
         }
         {
@@ -1385,8 +1238,15 @@ template <int N1> struct BandL {
         }
         {
             ProfileScope prof_(MWG_KERNEL_REDUCE);
-            hipLaunchKernelGGL(k_reduce_units<N1>, dim3(L, (8 * N3 + 255) / 256), dim3(256), 0, 0, dev.segs, dev.node_seg, lvl->g_off, uscan,
-                               w.partial.as<double>());
+            const dim3 rgrid(L, (8 * N3 + 255) / 256);
+            if (!waves)
+                hipLaunchKernelGGL(k_reduce_units<N1>, rgrid, dim3(256), 0, 0, dev.segs, dev.node_seg, lvl->g_off, uscan, w.partial.as<double>());
+            else if (precision == MWG_PREC_FP64)
+                hipLaunchKernelGGL((k_reduce_waves<N1, MWG_PREC_FP64>), rgrid, dim3(256), 0, 0, dev.segs, dev.node_seg, lvl->g_off, uscan,
+                                   w.partial.as<double>());
+            else
+                hipLaunchKernelGGL((k_reduce_waves<N1, MWG_PREC_FP32>), rgrid, dim3(256), 0, 0, dev.segs, dev.node_seg, lvl->g_off, uscan,
+                                   w.partial.as<double>());
             MWG_LAUNCHED();
             hipLaunchKernelGGL(k_level_norms<N1>, dim3(L), dim3(kThreads), 0, 0, dev.segs, dev.node_seg, lvl->g_off, lvl->g_norms);
             MWG_LAUNCHED();
