@@ -267,9 +267,9 @@ class FunctionTree:
         """(idx[N,5] = scale, lx, ly, lz, is_end; coefs[N, 8 (k+1)^3] or None; norms[N, 9])."""
         n = self.getNNodes()
         kp1_d = (self.mra.order + 1) ** 3
-        idx = np.zeros((n, 5), dtype=np.int32)
-        coefs = np.zeros((n, 8 * kp1_d)) if with_coefs else None
-        norms = np.zeros((n, 9))
+        idx = np.empty((n, 5), dtype=np.int32)
+        coefs = np.empty((n, 8 * kp1_d)) if with_coefs else None
+        norms = np.empty((n, 9))
         got = lib().mrcpp_tree_export(self._h, _p(idx, _ip), _p(coefs) if with_coefs else None, _p(norms))
         if got < 0:
             raise MRCPPError(lib().mrcpp_last_error().decode())

@@ -99,15 +99,14 @@ int mrcpp_tree_export(void *tree, int *idx, double *coefs, double *norms) {
     int n = -1;
     int rc = guarded([&] {
         auto &t = *static_cast<FunctionTree<3> *>(tree);
-        auto &s = coefs ? t.nodes() : t.topology();
+        auto &s = t.topology();
         auto all = detail::real_nodes(s);
-        const int nc = s.ncoef();
+        if (coefs) t.copyCoefs(all, coefs);
         for (size_t i = 0; i < all.size(); i++) {
             const int u = all[i];
             idx[5 * i] = s.scale(u);
             for (int d = 0; d < 3; d++) idx[5 * i + 1 + d] = s.transl(u)[d];
             idx[5 * i + 4] = s.isEnd(u) ? 1 : 0;
-            if (coefs) std::memcpy(coefs + (size_t)i * nc, s.coefs(u), sizeof(double) * nc);
             if (norms) {
                 for (int c = 0; c < 8; c++) norms[9 * i + c] = s.compNorm(u, c);
                 norms[9 * i + 8] = s.squareNorm(u);

@@ -4,6 +4,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <omp.h>
 #include <map>
 #include <mutex>
 
@@ -11,6 +12,30 @@
 
 namespace mrcpp {
 namespace device {
+
+void download_rows(const double *src, size_t row_doubles, const std::vector<double *> &dst) {
+    struct Job {
+        const std::vector<double *> &dst;
+        size_t row; // bytes
+        int threads;
+    } job{dst, sizeof(double) * row_doubles, std::max(1, omp_get_max_threads() - 2)}; // two cores left to the runtime's threads
+    const size_t bytes = dst.size() * job.row;
+    // whole rows per piece, four pieces or more where the rows fill them (the
+    // host then works on one while the link carries the next)
+    const size_t target = std::min<size_t>(std::max<size_t>(bytes / 4, size_t(512) << 10), size_t(4) << 20);
+    const size_t piece = std::max<size_t>(target / job.row, 1) * job.row;
+    auto place = [](void *ctx, const void *piece, size_t offset, size_t size) {
+        const Job &j = *static_cast<const Job *>(ctx);
+        const long first = (long)(offset / j.row), n = (long)(size / j.row);
+        // a thread's share is at least 64 KiB: waking one costs about as much
+        const int threads = std::min<long>(j.threads, std::max<long>(1, (long)(size >> 16)));
+#pragma omp parallel for schedule(static) num_threads(threads) if (threads > 1)
+        for (long i = 0; i < n; i++)
+            if (double *d = j.dst[first + i]) std::memcpy(d, static_cast<const char *>(piece) + i * j.row, j.row);
+    };
+    check(mwg_download_stream(src, bytes, piece, place, &job), "download");
+}
+
 
 void check(mwg_status s, const char *what) {
     if (s != MWG_OK) throw Error(std::string(what) + ": " + mwg_last_error());

@@ -78,6 +78,11 @@ private:
     size_t cap_ = 0;
 };
 
+// Rows of device memory (row i: row_doubles at src + i row_doubles) to
+// dst[i] each (null: skipped), the host threads placing one piece while the
+// next are on the link.
+void download_rows(const double *src, size_t row_doubles, const std::vector<double *> &dst);
+
 // Page-locked host buffer, grown on demand (contents are not kept).
 template <typename T> class PinnedArray {
 public:

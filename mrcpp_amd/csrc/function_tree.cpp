@@ -29,11 +29,22 @@ int FunctionTree<3>::getNEndNodes() const { return (int)detail::end_nodes(*store
 void FunctionTree<3>::syncHost() {
     if (!host_stale_) return;
     detail::NodeStore<3> &s = *store_;
-    const size_t nc = s.ncoef();
-    std::vector<double> buf((size_t)s.size() * nc);
-    dev_coef_.download(buf.data(), buf.size());
-    for (int u = 0; u < s.size(); u++) std::memcpy(s.coefs(u), buf.data() + (size_t)u * nc, sizeof(double) * nc);
+    std::vector<double *> rows(s.size());
+    for (int u = 0; u < s.size(); u++) rows[u] = s.coefs(u);
+    device::download_rows(dev_coef_.get(), s.ncoef(), rows);
     host_stale_ = false;
+}
+
+void FunctionTree<3>::copyCoefs(const std::vector<int> &order, double *out) {
+    detail::NodeStore<3> &s = *store_;
+    const size_t nc = s.ncoef();
+    if (!host_stale_) {
+        for (size_t i = 0; i < order.size(); i++) std::memcpy(out + i * nc, s.coefs(order[i]), sizeof(double) * nc);
+        return;
+    }
+    std::vector<double *> rows(s.size(), nullptr);
+    for (size_t i = 0; i < order.size(); i++) rows[order[i]] = out + i * nc;
+    device::download_rows(dev_coef_.get(), nc, rows);
 }
 
 detail::NodeStore<3> &FunctionTree<3>::nodes() {

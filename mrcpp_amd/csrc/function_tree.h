@@ -70,6 +70,9 @@ public:
         mirror_.reset();
     }
     bool hostStale() const { return host_stale_; }
+    // Coefficients of the nodes `order` to out, 8 (k+1)^3 each: straight from
+    // the device when they live there (the host store is left as it is)
+    void copyCoefs(const std::vector<int> &order, double *out);
     void syncHost();
     // device mirror used when this tree is the input of apply
     device::TreeMirror &inputMirror();

@@ -413,6 +413,41 @@ mwg_status mwg_download_many(int n, void *const *dst, const void *const *src, co
     return MWG_OK;
 }
 
+// Four pieces share the landing buffer: the link carries one while the caller
+// takes another (a copy engine's 4 MiB take 82 us, the same bytes to the
+// caller's fresh pages about as long on the host's threads).
+mwg_status mwg_download_stream(const void *src, size_t bytes, size_t piece_bytes, mwg_sink sink, void *ctx) {
+    constexpr int kPieces = 4;
+    if (!bytes) return MWG_OK;
+    if (!src || !sink) return fail(MWG_ERR_ARG, "null pointer");
+    if (piece_bytes == 0 || piece_bytes > kStageMaxCopy / kPieces) return fail(MWG_ERR_ARG, "piece size out of range");
+    if (mwg_status s = ensure_landing(); s != MWG_OK) return s;
+    static hipEvent_t landed[kPieces];
+    static bool created = false;
+    if (!created) {
+        for (hipEvent_t &e : landed) MWG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        created = true;
+    }
+    const size_t n = (bytes + piece_bytes - 1) / piece_bytes;
+    auto size_of = [&](size_t i) { return std::min(piece_bytes, bytes - i * piece_bytes); };
+    auto buffer = [&](size_t i) { return g_landing + (i % kPieces) * piece_bytes; };
+    auto request = [&](size_t i) -> mwg_status {
+        MWG_HIP(hipMemcpyAsync(buffer(i), static_cast<const unsigned char *>(src) + i * piece_bytes, size_of(i), hipMemcpyDeviceToHost, 0));
+        MWG_HIP(hipEventRecord(landed[i % kPieces], 0));
+        return MWG_OK;
+    };
+    for (size_t i = 0; i < std::min<size_t>(n, kPieces); i++)
+        if (mwg_status s = request(i); s != MWG_OK) return s;
+    for (size_t i = 0; i < n; i++) {
+        MWG_HIP(hipEventSynchronize(landed[i % kPieces]));
+        sink(ctx, buffer(i), i * piece_bytes, size_of(i));
+        if (i + kPieces < n)
+            if (mwg_status s = request(i + kPieces); s != MWG_OK) return s;
+    }
+    g_stage_used = 0; // the null stream has drained
+    return MWG_OK;
+}
+
 mwg_status mwg_copy(void *dst, const void *src, size_t bytes) {
     if (!bytes) return MWG_OK;
     if (!dst || !src) return fail(MWG_ERR_ARG, "null pointer");
