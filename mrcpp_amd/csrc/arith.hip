@@ -2,7 +2,7 @@
 // (AdditionCalculator::calcNode, src/treebuilders/AdditionCalculator.h:45-70;
 // MultiplicationCalculator::calcNode, src/treebuilders/MultiplicationCalculator.h:45-83).
 //
-// One 256-thread workgroup per output node.  A sum reads the operands' nodes
+// One workgroup per output node.  A sum reads the operands' nodes
 // and writes their linear combination.  A product takes each operand's node
 // through its reconstruction to the 8 children's scaling blocks and the
 // coefficient -> value maps (MWNode::mwTransform(Reconstruction),
@@ -19,18 +19,30 @@ namespace mwgdev {
 namespace {
 
 // out(r, j) = sum_i in(i, r) M(i, j) for each of the 8 blocks (the host's
-// math_utils::apply_filter view, in N1 x N1^2 column-major), padded LDS layout.
+// math_utils::apply_filter view, in N1 x N1^2 column-major), padded LDS layout;
+// 2 x 2 outputs per thread (SmallTile).
 template <int N1> __device__ inline void map_pass(double *out, const double *in, const double *M) {
+    using P = SmallTile<N1>;
     constexpr int N2 = N1 * N1, N3 = N2 * N1;
-    for (int o = threadIdx.x; o < 8 * N3; o += kThreads) {
-        const int t = o / N3, e = o % N3;
-        const int r = e % N2, j = e / N2;
-        const double *x = in + pad<N1>(t * N3 + N1 * r);
-        const double *m = M + N1 * j;
-        double s = 0.0;
+    for (int t = threadIdx.x; t < P::TILES; t += kPassThreads) {
+        const int blk = t / (P::JG * P::RB), j0 = ((t / P::RB) % P::JG) * 2, rb = t % P::RB;
+        double s[2][2] = {{0.0, 0.0}, {0.0, 0.0}};
+#pragma unroll 2
+        for (int i = 0; i < N1; i++) {
+            double x[2], m[2];
 #pragma unroll
-        for (int i = 0; i < N1; i++) s += x[i] * m[i];
-        out[pad<N1>(o)] = s;
+            for (int q = 0; q < 2; q++) x[q] = in[pad<N1>(blk * N3 + N1 * (rb + q * P::RB) + i)];
+#pragma unroll
+            for (int c = 0; c < 2; c++) m[c] = M[N1 * (j0 + c) + i];
+#pragma unroll
+            for (int c = 0; c < 2; c++)
+#pragma unroll
+                for (int q = 0; q < 2; q++) s[c][q] += x[q] * m[c];
+        }
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+            for (int q = 0; q < 2; q++) out[pad<N1>(blk * N3 + (j0 + c) * N2 + rb + q * P::RB)] = s[c][q];
     }
 }
 
@@ -39,13 +51,62 @@ template <int N1> __device__ inline void load_operand(double *dst, const double 
     constexpr int N3 = N1 * N1 * N1;
     const bool gen = off < 0;
     const long long base = gen ? -off - 1 : off;
-    for (int o = threadIdx.x; o < 8 * N3; o += kThreads) dst[pad<N1>(o)] = (gen && o >= N3) ? 0.0 : pool[base + o];
+    for (int o = threadIdx.x; o < 8 * N3; o += kPassThreads) dst[pad<N1>(o)] = (gen && o >= N3) ? 0.0 : pool[base + o];
 }
 
+// coefs_o = 0; coefs_o += c_i coefs_i, operand by operand, and the norms (the
+// order of block_norms).  Bound by the reads' latency: every load of a thread's
+// values is in flight at once and nothing goes through LDS, so eight workgroups
+// share a CU (one kernel for sums and products held two; 273 order-7 nodes a
+// launch: 46 -> 13 us).
 template <int N1>
-__global__ __launch_bounds__(kThreads) void k_combine(mwg_combine cb, const long long *in_off, const int *scale, const long long *out_off,
-                                                      double *out, double *norms) {
-    constexpr int N2 = N1 * N1, N3 = N2 * N1, PT = (8 * N3 + kThreads - 1) / kThreads;
+__global__ __launch_bounds__(kThreads) void k_sum(mwg_combine cb, const long long *in_off, const long long *out_off, double *out, double *norms) {
+    constexpr int N3 = N1 * N1 * N1, PT = (8 * N3 + kThreads - 1) / kThreads;
+    __shared__ double red[8 * (kThreads / 64)];
+    const int k = blockIdx.x;
+    const auto offs = ro(in_off) + (size_t)k * cb.nin;
+    double *dst = out + out_off[k];
+    double s[PT];
+#pragma unroll
+    for (int p = 0; p < PT; p++) s[p] = 0.0;
+    for (int i = 0; i < cb.nin; i++) {
+        const long long off = offs[i];
+        const bool gen = off < 0;
+        const double *src = cb.pool[i] + (gen ? -off - 1 : off);
+        const double c = cb.c[i];
+        double v[PT];
+#pragma unroll
+        for (int p = 0; p < PT; p++) {
+            const int o = threadIdx.x + kThreads * p;
+            v[p] = o < (gen ? N3 : 8 * N3) ? src[o] : 0.0;
+        }
+#pragma unroll
+        for (int p = 0; p < PT; p++) s[p] += c * v[p];
+    }
+    double ss[8];
+#pragma unroll
+    for (int t = 0; t < 8; t++) ss[t] = 0.0;
+#pragma unroll
+    for (int p = 0; p < PT; p++) {
+        const int o = threadIdx.x + kThreads * p;
+        if (o < 8 * N3) {
+            dst[o] = s[p];
+#pragma unroll
+            for (int t = 0; t < 8; t++)
+                if (o / N3 == t) ss[t] += s[p] * s[p];
+        }
+    }
+    norms_of_sums(ss, norms + (size_t)k * 9, red);
+}
+
+// Products: kPassThreads threads, 2 x 2 outputs each in every pass (a 256-thread
+// workgroup with 4 x 5 and single outputs: 162 -> 114 us a launch at order 9,
+// 43 -> 36 at order 5).  Bound by LDS reads, one a multiply-add, and the chain of
+// passes.
+template <int N1>
+__global__ __launch_bounds__(kPassThreads) void k_product(mwg_combine cb, const long long *in_off, const int *scale, const long long *out_off,
+                                                          double *out, double *norms) {
+    constexpr int N2 = N1 * N1, N3 = N2 * N1, PT = (8 * N3 + kPassThreads - 1) / kPassThreads;
     __shared__ double a[Lds<N1>::size], b[Lds<N1>::size];
     __shared__ double red[8 * (kThreads / 64)];
     __shared__ double cvm[N2], vcm[N2];
@@ -53,28 +114,11 @@ __global__ __launch_bounds__(kThreads) void k_combine(mwg_combine cb, const long
     const int k = blockIdx.x;
     const long long *offs = in_off + (size_t)k * cb.nin;
     double *dst = out + out_off[k];
-    if (cb.mode == 0) {
-        // coefs_o = 0; coefs_o += c_i coefs_i, operand by operand
-        for (int o = threadIdx.x; o < 8 * N3; o += kThreads) {
-            double s = 0.0;
-            for (int i = 0; i < cb.nin; i++) {
-                const long long off = offs[i];
-                const bool gen = off < 0;
-                const double v = gen ? (o < N3 ? cb.pool[i][-off - 1 + o] : 0.0) : cb.pool[i][off + o];
-                s += cb.c[i] * v;
-            }
-            a[pad<N1>(o)] = s;
-            dst[o] = s;
-        }
-        __syncthreads();
-        block_norms<N1, true>(a, norms + (size_t)k * 9, red);
-        return;
-    }
-    for (int i = threadIdx.x; i < N2; i += kThreads) {
+    for (int i = threadIdx.x; i < N2; i += kPassThreads) {
         cvm[i] = cb.cvmap[i];
         vcm[i] = cb.vcmap[i];
     }
-    stage_filters<N1>(sfl, cb.filters, 8);
+    for (int i = threadIdx.x; i < 8 * N2; i += kPassThreads) sfl[i] = cb.filters[i];
     const int n = scale[k];
     double sfp = cb.sf[0] * cb.sf[1] * cb.sf[2];
     if (sfp <= kMachineZero) sfp = 1.0;
@@ -87,11 +131,11 @@ __global__ __launch_bounds__(kThreads) void k_combine(mwg_combine cb, const long
         __syncthreads(); // the previous operand's values are consumed
         load_operand<N1>(a, cb.pool[i], offs[i]);
         __syncthreads();
-        mw_pass<N1>(b, a, sfl, 4, 0);
+        small_pass<N1>(b, a, sfl, 4, 0);
         __syncthreads();
-        mw_pass<N1>(a, b, sfl, 4, 1);
+        small_pass<N1>(a, b, sfl, 4, 1);
         __syncthreads();
-        mw_pass<N1>(b, a, sfl, 4, 2);
+        small_pass<N1>(b, a, sfl, 4, 2);
         __syncthreads();
         map_pass<N1>(a, b, cvm);
         __syncthreads();
@@ -102,14 +146,14 @@ __global__ __launch_bounds__(kThreads) void k_combine(mwg_combine cb, const long
         const double ci = cb.c[i];
 #pragma unroll
         for (int p = 0; p < PT; p++) {
-            const int o = threadIdx.x + kThreads * p;
+            const int o = threadIdx.x + kPassThreads * p;
             if (o < 8 * N3) val[p] = val[p] * (ci * (fwd * a[pad<N1>(o)]));
         }
     }
     __syncthreads();
 #pragma unroll
     for (int p = 0; p < PT; p++) {
-        const int o = threadIdx.x + kThreads * p;
+        const int o = threadIdx.x + kPassThreads * p;
         if (o < 8 * N3) a[pad<N1>(o)] = val[p];
     }
     __syncthreads();
@@ -120,15 +164,15 @@ __global__ __launch_bounds__(kThreads) void k_combine(mwg_combine cb, const long
     __syncthreads();
     map_pass<N1>(b, a, vcm);
     __syncthreads();
-    for (int o = threadIdx.x; o < 8 * N3; o += kThreads) b[pad<N1>(o)] = bwd * b[pad<N1>(o)];
+    for (int o = threadIdx.x; o < 8 * N3; o += kPassThreads) b[pad<N1>(o)] = bwd * b[pad<N1>(o)];
     __syncthreads();
-    mw_pass<N1>(a, b, sfl, 0, 0);
+    small_pass<N1>(a, b, sfl, 0, 0);
     __syncthreads();
-    mw_pass<N1>(b, a, sfl, 0, 1);
+    small_pass<N1>(b, a, sfl, 0, 1);
     __syncthreads();
-    mw_pass<N1>(a, b, sfl, 0, 2);
+    small_pass<N1>(a, b, sfl, 0, 2);
     __syncthreads();
-    for (int o = threadIdx.x; o < 8 * N3; o += kThreads) dst[o] = a[pad<N1>(o)];
+    for (int o = threadIdx.x; o < 8 * N3; o += kPassThreads) dst[o] = a[pad<N1>(o)];
     block_norms<N1, true>(a, norms + (size_t)k * 9, red);
 }
 
@@ -136,7 +180,10 @@ template <int N1> struct CombineL {
     static mwg_status run(const mwg_combine *cb, const long long *in_off, const int *scale, const long long *out_off, double *out, double *norms,
                           int count) {
         ProfileScope prof_(MWG_KERNEL_ARITH);
-        hipLaunchKernelGGL(k_combine<N1>, dim3(count), dim3(kThreads), 0, 0, *cb, in_off, scale, out_off, out, norms);
+        if (cb->mode == 0)
+            hipLaunchKernelGGL(k_sum<N1>, dim3(count), dim3(kThreads), 0, 0, *cb, in_off, out_off, out, norms);
+        else
+            hipLaunchKernelGGL(k_product<N1>, dim3(count), dim3(kPassThreads), 0, 0, *cb, in_off, scale, out_off, out, norms);
         MWG_LAUNCHED();
         return MWG_OK;
     }

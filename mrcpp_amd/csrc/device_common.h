@@ -267,26 +267,84 @@ __device__ inline void mw_pass_add_children(double *coef, long long child_off, l
     }
 }
 
-// Component norms of 8 blocks, written to nrm[0..8] (8 norms + square norm);
-// PAD: c in the padded LDS layout.
-template <int N1, bool PAD = false> __device__ inline void block_norms(const double *c, double *nrm, double *red) {
-    constexpr int N3 = N1 * N1 * N1;
-    double ss[8];
+// The generation, top-down, bottom-up and product passes are latency-bound for
+// the few nodes of a launch: their workgroups have kPassThreads threads, each
+// forming a 2 x 2 register tile of a pass (the same per-output sum, over i in
+// increasing order, as the 4 x 4 tiles of mw_pass, so the same results).
+constexpr int kPassThreads = 1024;
+template <int N1> struct SmallTile {
+    static constexpr int N2 = N1 * N1, J = 2, R = 2, RB = N2 / R, JG = N1 / J, TILES = 8 * JG * RB;
+    static_assert(N1 % J == 0 && N2 % R == 0, "small pass tile shape");
+};
+template <int N1>
+__device__ __forceinline__ void small_tile(const double *in, const double *filt, int dir_base, int dim, int t, int &gt, int &j0, int &rb, double (&s0)[2][2],
+                                           double (&s1)[2][2]) {
+    using P = SmallTile<N1>;
+    constexpr int N2 = P::N2, N3 = N2 * N1, J = P::J, R = P::R, RB = P::RB;
+    gt = t / (P::JG * RB);
+    j0 = ((t / RB) % P::JG) * J;
+    rb = t % RB;
+    const int bit = 1 << dim;
+    const int ft0 = gt & ~bit, ft1 = gt | bit;
+    const double *F0 = filt + (size_t)(dir_base + 2 * ((gt >> dim) & 1) + 0) * N2 + N1 * j0;
+    const double *F1 = filt + (size_t)(dir_base + 2 * ((gt >> dim) & 1) + 1) * N2 + N1 * j0;
 #pragma unroll
-    for (int t = 0; t < 8; t++) ss[t] = 0.0;
-    for (int o = threadIdx.x; o < 8 * N3; o += kThreads) {
-        const double v = c[PAD ? pad<N1>(o) : o];
-        ss[o / N3] += v * v;
-    }
+    for (int p = 0; p < J; p++)
 #pragma unroll
-    for (int t = 0; t < 8; t++) {
-        double v = ss[t];
-        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-        ss[t] = v;
+        for (int q = 0; q < R; q++) {
+            s0[p][q] = 0.0;
+            s1[p][q] = 0.0;
+        }
+#pragma unroll 2
+    for (int i = 0; i < N1; i++) {
+        double x0[R], x1[R], f0[J], f1[J];
+#pragma unroll
+        for (int q = 0; q < R; q++) {
+            x0[q] = in[pad<N1>(ft0 * N3 + N1 * (rb + q * RB) + i)];
+            x1[q] = in[pad<N1>(ft1 * N3 + N1 * (rb + q * RB) + i)];
+        }
+#pragma unroll
+        for (int p = 0; p < J; p++) {
+            f0[p] = F0[N1 * p + i];
+            f1[p] = F1[N1 * p + i];
+        }
+#pragma unroll
+        for (int p = 0; p < J; p++)
+#pragma unroll
+            for (int q = 0; q < R; q++) {
+                s0[p][q] += x0[q] * f0[p];
+                s1[p][q] += x1[q] * f1[p];
+            }
     }
+}
+template <int N1> __device__ __forceinline__ void small_pass(double *out, const double *in, const double *filt, int dir_base, int dim) {
+    using P = SmallTile<N1>;
+    constexpr int N2 = P::N2, N3 = N2 * N1;
+    for (int t = threadIdx.x; t < P::TILES; t += kPassThreads) {
+        double s0[2][2], s1[2][2];
+        int gt, j0, rb;
+        small_tile<N1>(in, filt, dir_base, dim, t, gt, j0, rb, s0, s1);
+#pragma unroll
+        for (int p = 0; p < 2; p++)
+#pragma unroll
+            for (int q = 0; q < 2; q++) out[pad<N1>(gt * N3 + (j0 + p) * N2 + rb + q * P::RB)] = s0[p][q] + s1[p][q];
+    }
+}
+// Component norms from the first kThreads threads' sums of squares ss[8],
+// written to nrm[0..8] (8 norms + square norm): lanes by a fixed tree, waves in
+// order.  Every thread of the workgroup must call.
+__device__ inline void norms_of_sums(double (&ss)[8], double *nrm, double *red) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (lane == 0)
-        for (int t = 0; t < 8; t++) red[wave * 8 + t] = ss[t];
+    if (threadIdx.x < kThreads) {
+#pragma unroll
+        for (int t = 0; t < 8; t++) {
+            double v = ss[t];
+            for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+            ss[t] = v;
+        }
+        if (lane == 0)
+            for (int t = 0; t < 8; t++) red[wave * 8 + t] = ss[t];
+    }
     __syncthreads();
     if (threadIdx.x == 0) {
         double tot = 0.0;
@@ -300,6 +358,20 @@ template <int N1, bool PAD = false> __device__ inline void block_norms(const dou
         nrm[8] = tot;
     }
     __syncthreads();
+}
+
+// Component norms of 8 blocks (PAD: c in the padded LDS layout).
+template <int N1, bool PAD = false> __device__ inline void block_norms(const double *c, double *nrm, double *red) {
+    constexpr int N3 = N1 * N1 * N1;
+    double ss[8];
+#pragma unroll
+    for (int t = 0; t < 8; t++) ss[t] = 0.0;
+    if (threadIdx.x < kThreads)
+        for (int o = threadIdx.x; o < 8 * N3; o += kThreads) {
+            const double v = c[PAD ? pad<N1>(o) : o];
+            ss[o / N3] += v * v;
+        }
+    norms_of_sums(ss, nrm, red);
 }
 
 } // namespace mwgdev
