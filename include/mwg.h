@@ -458,8 +458,8 @@ mwg_status mwg_operator_nodes(int kp1, const double *left, const double *right, 
  * >= 0: operand i's node k (8 blocks) at that offset in pool[i]; < 0: a
  * generated node, its scaling block at -in_off - 1 (wavelet blocks zero).
  * scale[k] is the node's scale, out_off[k] its offset in out; norms[9 k] the 8
- * component norms and the square norm.  No fused multiply-add: the host's
- * order of operations. */
+ * component norms and the square norm.  Sums take no fused multiply-add: the
+ * host's order of operations. */
 #define MWG_MAX_OPERANDS 8
 typedef struct {
     int kp1;

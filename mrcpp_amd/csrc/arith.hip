@@ -7,52 +7,16 @@
 // through its reconstruction to the 8 children's scaling blocks and the
 // coefficient -> value maps (MWNode::mwTransform(Reconstruction),
 // MWNode::cvTransform(Forward), src/trees/MWNode.cpp:448-594) in LDS,
-// multiplies the values into registers, then maps back and compresses.  The
-// file is compiled without fused multiply-adds and every sum runs in the
-// host's order, so the results equal the host formation.
+// multiplies the values in registers, then maps back and compresses.  The
+// file is compiled without fused multiply-adds: a sum's nodes equal the host
+// formation.
 #pragma clang fp contract(off)
 
-#include "device_common.h"
+#include "mw_passes.h"
 
 namespace mwgdev {
 
 namespace {
-
-// out(r, j) = sum_i in(i, r) M(i, j) for each of the 8 blocks (the host's
-// math_utils::apply_filter view, in N1 x N1^2 column-major), padded LDS layout;
-// 2 x 2 outputs per thread (SmallTile).
-template <int N1> __device__ inline void map_pass(double *out, const double *in, const double *M) {
-    using P = SmallTile<N1>;
-    constexpr int N2 = N1 * N1, N3 = N2 * N1;
-    for (int t = threadIdx.x; t < P::TILES; t += kPassThreads) {
-        const int blk = t / (P::JG * P::RB), j0 = ((t / P::RB) % P::JG) * 2, rb = t % P::RB;
-        double s[2][2] = {{0.0, 0.0}, {0.0, 0.0}};
-#pragma unroll 2
-        for (int i = 0; i < N1; i++) {
-            double x[2], m[2];
-#pragma unroll
-            for (int q = 0; q < 2; q++) x[q] = in[pad<N1>(blk * N3 + N1 * (rb + q * P::RB) + i)];
-#pragma unroll
-            for (int c = 0; c < 2; c++) m[c] = M[N1 * (j0 + c) + i];
-#pragma unroll
-            for (int c = 0; c < 2; c++)
-#pragma unroll
-                for (int q = 0; q < 2; q++) s[c][q] += x[q] * m[c];
-        }
-#pragma unroll
-        for (int c = 0; c < 2; c++)
-#pragma unroll
-            for (int q = 0; q < 2; q++) out[pad<N1>(blk * N3 + (j0 + c) * N2 + rb + q * P::RB)] = s[c][q];
-    }
-}
-
-// operand i's node k into LDS (a generated node: scaling block, zero wavelets)
-template <int N1> __device__ inline void load_operand(double *dst, const double *pool, long long off) {
-    constexpr int N3 = N1 * N1 * N1;
-    const bool gen = off < 0;
-    const long long base = gen ? -off - 1 : off;
-    for (int o = threadIdx.x; o < 8 * N3; o += kPassThreads) dst[pad<N1>(o)] = (gen && o >= N3) ? 0.0 : pool[base + o];
-}
 
 // coefs_o = 0; coefs_o += c_i coefs_i, operand by operand, and the norms (the
 // order of block_norms).  Bound by the reads' latency: every load of a thread's
@@ -99,81 +63,58 @@ __global__ __launch_bounds__(kThreads) void k_sum(mwg_combine cb, const long lon
     norms_of_sums(ss, norms + (size_t)k * 9, red);
 }
 
-// Products: kPassThreads threads, 2 x 2 outputs each in every pass (a 256-thread
-// workgroup with 4 x 5 and single outputs: 162 -> 114 us a launch at order 9,
-// 43 -> 36 at order 5).  Bound by LDS reads, one a multiply-add, and the chain of
-// passes.
+// Products.  Each pass takes its direction's filters and its map between
+// coefficients and values, so an operand takes three passes and the way back
+// three (before, six each on the vector units: 114 -> 46 us a launch at order 9,
+// 36 -> 18 at order 5), and the values are multiplied in the registers the
+// third pass leaves them in.  Bound by the chain of loads, passes and barriers of a node.
 template <int N1>
-__global__ __launch_bounds__(kPassThreads) void k_product(mwg_combine cb, const long long *in_off, const int *scale, const long long *out_off,
-                                                          double *out, double *norms) {
-    constexpr int N2 = N1 * N1, N3 = N2 * N1, PT = (8 * N3 + kPassThreads - 1) / kPassThreads;
-    __shared__ double a[Lds<N1>::size], b[Lds<N1>::size];
-    __shared__ double red[8 * (kThreads / 64)];
-    __shared__ double cvm[N2], vcm[N2];
-    __shared__ double sfl[8 * N2];
+__global__ __launch_bounds__(MwShape<N1>::THREADS, MwShape<N1>::OCC) void k_product(mwg_combine cb, const long long *in_off, const int *scale, const long long *out_off,
+                                                                  double *out, double *norms) {
+    using P = MwShape<N1>;
+    constexpr int T = P::T;
+    __shared__ double a[P::SIZE], b[P::SIZE];
+    __shared__ double cvs[MwMap<N1>::STORE], vcs[MwMap<N1>::STORE], red[8];
     const int k = blockIdx.x;
-    const long long *offs = in_off + (size_t)k * cb.nin;
-    double *dst = out + out_off[k];
-    for (int i = threadIdx.x; i < N2; i += kPassThreads) {
-        cvm[i] = cb.cvmap[i];
-        vcm[i] = cb.vcmap[i];
-    }
-    for (int i = threadIdx.x; i < 8 * N2; i += kPassThreads) sfl[i] = cb.filters[i];
+    const auto offs = ro(in_off) + (size_t)k * cb.nin;
+    MwMap<N1> cv, vc;
+    cv.load(cb.cvmap, cvs);
+    if constexpr (MwMap<N1>::LDS) vc.load(cb.vcmap, vcs);
     const int n = scale[k];
     double sfp = cb.sf[0] * cb.sf[1] * cb.sf[2];
     if (sfp <= kMachineZero) sfp = 1.0;
     const double two_fac = ldexp(1.0, 3 * (n + 1)) / sfp;
     const double fwd = sqrt(two_fac), bwd = sqrt(1.0 / two_fac);
-    double val[PT];
+    double val[P::PER][T];
 #pragma unroll
-    for (int p = 0; p < PT; p++) val[p] = 1.0;
-    for (int i = 0; i < cb.nin; i++) {
-        __syncthreads(); // the previous operand's values are consumed
-        load_operand<N1>(a, cb.pool[i], offs[i]);
-        __syncthreads();
-        small_pass<N1>(b, a, sfl, 4, 0);
-        __syncthreads();
-        small_pass<N1>(a, b, sfl, 4, 1);
-        __syncthreads();
-        small_pass<N1>(b, a, sfl, 4, 2);
-        __syncthreads();
-        map_pass<N1>(a, b, cvm);
-        __syncthreads();
-        map_pass<N1>(b, a, cvm);
-        __syncthreads();
-        map_pass<N1>(a, b, cvm);
-        __syncthreads();
-        const double ci = cb.c[i];
+    for (int q = 0; q < P::PER; q++)
 #pragma unroll
-        for (int p = 0; p < PT; p++) {
-            const int o = threadIdx.x + kPassThreads * p;
-            if (o < 8 * N3) val[p] = val[p] * (ci * (fwd * a[pad<N1>(o)]));
+        for (int J = 0; J < T; J++) val[q][J] = 1.0;
+    __syncthreads();
+    {
+        MwMatrix<N1> M;
+        M.filters(cb.filters, 4);
+        for (int i = 0; i < cb.nin; i++) {
+            const long long off = offs[i];
+            const bool gen = off < 0; // a generated node: scaling block, zero wavelets
+            const double *src = cb.pool[i] + (gen ? -off - 1 : off);
+            mw_pass<N1, 0, MW_MAP_AFTER>(
+                M, [&](int t, int r, int e) { return gen && t != 0 ? 0.0 : src[t * P::N3 + N1 * r + e]; },
+                [&](int, int, int t, int j, int r, double v) { a[P::at_out(t, j, r)] = v; }, cv);
+            __syncthreads();
+            mw_pass_lds<N1, 1, MW_MAP_AFTER>(b, a, M, cv);
+            __syncthreads();
+            const double ci = cb.c[i];
+            mw_pass<N1, 2, MW_MAP_AFTER>(
+                M, [&](int t, int r, int e) { return b[P::at(t, r, e)]; },
+                [&](int q, int J, int, int, int, double v) { val[q][J] *= ci * (fwd * v); }, cv);
         }
     }
+    if constexpr (!MwMap<N1>::LDS) vc.load(cb.vcmap, vcs);
+    // the values (where the third pass left them) to LDS
+    mw_own<N1, 2>([&](int q, int J, int t, int j, int r) { a[P::at_out(t, j, r)] = bwd * val[q][J]; });
     __syncthreads();
-#pragma unroll
-    for (int p = 0; p < PT; p++) {
-        const int o = threadIdx.x + kPassThreads * p;
-        if (o < 8 * N3) a[pad<N1>(o)] = val[p];
-    }
-    __syncthreads();
-    // values -> scaling coefficients of the children, then compression
-    map_pass<N1>(b, a, vcm);
-    __syncthreads();
-    map_pass<N1>(a, b, vcm);
-    __syncthreads();
-    map_pass<N1>(b, a, vcm);
-    __syncthreads();
-    for (int o = threadIdx.x; o < 8 * N3; o += kPassThreads) b[pad<N1>(o)] = bwd * b[pad<N1>(o)];
-    __syncthreads();
-    small_pass<N1>(a, b, sfl, 0, 0);
-    __syncthreads();
-    small_pass<N1>(b, a, sfl, 0, 1);
-    __syncthreads();
-    small_pass<N1>(a, b, sfl, 0, 2);
-    __syncthreads();
-    for (int o = threadIdx.x; o < 8 * N3; o += kPassThreads) dst[o] = a[pad<N1>(o)];
-    block_norms<N1, true>(a, norms + (size_t)k * 9, red);
+    mw_values_to_node<N1>(a, b, cb.filters, vc, out + out_off[k], norms + (size_t)k * 9, red);
 }
 
 template <int N1> struct CombineL {
@@ -183,7 +124,7 @@ template <int N1> struct CombineL {
         if (cb->mode == 0)
             hipLaunchKernelGGL(k_sum<N1>, dim3(count), dim3(kThreads), 0, 0, *cb, in_off, out_off, out, norms);
         else
-            hipLaunchKernelGGL(k_product<N1>, dim3(count), dim3(kPassThreads), 0, 0, *cb, in_off, scale, out_off, out, norms);
+            hipLaunchKernelGGL(k_product<N1>, dim3(count), dim3(MwShape<N1>::THREADS), 0, 0, *cb, in_off, scale, out_off, out, norms);
         MWG_LAUNCHED();
         return MWG_OK;
     }

@@ -155,181 +155,6 @@ template <template <int> class Launcher, typename... Args> mwg_status dispatch(i
     }
 }
 
-// LDS layout of a node's 8 blocks in the transform kernels: one padding
-// double after every row of N1 values, so the rows that the lanes of a pass
-// read (N1 apart without padding: lanes on few banks) spread over the banks.
-template <int N1> struct Lds {
-    static constexpr int N3 = N1 * N1 * N1, size = 8 * N3 + 8 * N3 / N1;
-};
-template <int N1> __device__ __forceinline__ int pad(int o) { return o + o / N1; }
-
-// The first `count` filter matrices (N1 x N1 each) of a filter bank into LDS:
-// the passes read every filter element once per output, from LDS rather than
-// through the vector memory path.
-template <int N1> __device__ inline void stage_filters(double *dst, const double *filt, int count) {
-    for (int i = threadIdx.x; i < count * N1 * N1; i += kThreads) dst[i] = filt[i];
-}
-
-// One pass of the separable 3D multiwavelet transform over 8 blocks in LDS
-// (padded layout).
-// dir_base 0: compression sub-filters, 4: reconstruction sub-filters (the
-// device filter array holds H0t,H1t,G0t,G1t then H0,G0,H1,G1).  out[gt] =
-// in[ft0]^T F(2 b + 0) + in[ft1]^T F(2 b + 1), ft0 < ft1 the two blocks that
-// agree with gt outside direction dim, b = bit dim of gt, in viewed
-// (N1 x N1^2) column-major (math_utils::apply_filter).
-// Register tiles of a pass: a thread forms J = N1/2 output columns j of R = 4
-// rows r (2 for N1 = 10, within the register budget), rows N2/R apart so that consecutive lanes read consecutive (padded)
-// rows; every input row element and filter element is read once per tile
-// instead of once per output.
-template <int N1> struct PassTile {
-    static constexpr int N2 = N1 * N1, J = N1 / 2, R = N1 >= 10 ? 2 : 4, RB = N2 / R, TILES = 8 * 2 * RB;
-    static_assert(N1 % 2 == 0 && N2 % R == 0, "pass tile shape");
-};
-
-// s0[p][q] = sum_i in[ft0][r_q][i] F0[j_p][i], s1 likewise with ft1 / F1, the
-// sum over i in increasing order (the order of MRCPP's apply_filter loops).
-template <int N1>
-__device__ inline void pass_tile(const double *in, const double *filt, int dir_base, int dim, int t, int &gt, int &j0, int &rb,
-                                 double (&s0)[N1 / 2][PassTile<N1>::R], double (&s1)[N1 / 2][PassTile<N1>::R]) {
-    using P = PassTile<N1>;
-    constexpr int N2 = P::N2, N3 = N2 * N1, J = P::J, R = P::R, RB = P::RB;
-    gt = t / (2 * RB);
-    j0 = ((t / RB) % 2) * J;
-    rb = t % RB;
-    const int bit = 1 << dim;
-    const int ft0 = gt & ~bit, ft1 = gt | bit;
-    const double *F0 = filt + (size_t)(dir_base + 2 * ((gt >> dim) & 1) + 0) * N2 + N1 * j0;
-    const double *F1 = filt + (size_t)(dir_base + 2 * ((gt >> dim) & 1) + 1) * N2 + N1 * j0;
-#pragma unroll
-    for (int p = 0; p < J; p++)
-#pragma unroll
-        for (int q = 0; q < R; q++) {
-            s0[p][q] = 0.0;
-            s1[p][q] = 0.0;
-        }
-#pragma unroll 2
-    for (int i = 0; i < N1; i++) {
-        double x0[R], x1[R], f0[J], f1[J];
-#pragma unroll
-        for (int q = 0; q < R; q++) {
-            x0[q] = in[pad<N1>(ft0 * N3 + N1 * (rb + q * RB) + i)];
-            x1[q] = in[pad<N1>(ft1 * N3 + N1 * (rb + q * RB) + i)];
-        }
-#pragma unroll
-        for (int p = 0; p < J; p++) {
-            f0[p] = F0[N1 * p + i];
-            f1[p] = F1[N1 * p + i];
-        }
-#pragma unroll
-        for (int p = 0; p < J; p++)
-#pragma unroll
-            for (int q = 0; q < R; q++) {
-                s0[p][q] += x0[q] * f0[p];
-                s1[p][q] += x1[q] * f1[p];
-            }
-    }
-}
-
-template <int N1> __device__ inline void mw_pass(double *out, const double *in, const double *filt, int dir_base, int dim) {
-    using P = PassTile<N1>;
-    constexpr int N2 = P::N2, N3 = N2 * N1;
-    for (int t = threadIdx.x; t < P::TILES; t += kThreads) {
-        double s0[P::J][P::R], s1[P::J][P::R];
-        int gt, j0, rb;
-        pass_tile<N1>(in, filt, dir_base, dim, t, gt, j0, rb, s0, s1);
-#pragma unroll
-        for (int p = 0; p < P::J; p++)
-#pragma unroll
-            for (int q = 0; q < P::R; q++) out[pad<N1>(gt * N3 + (j0 + p) * N2 + rb + q * P::RB)] = s0[p][q] + s1[p][q];
-    }
-}
-
-// Last reconstruction pass accumulating into the children's scaling blocks,
-// each of the two contributions added separately (in: padded LDS layout).
-template <int N1>
-__device__ inline void mw_pass_add_children(double *coef, long long child_off, long long stride, const double *in, const double *filt) {
-    using P = PassTile<N1>;
-    constexpr int N2 = P::N2;
-    for (int t = threadIdx.x; t < P::TILES; t += kThreads) {
-        double s0[P::J][P::R], s1[P::J][P::R];
-        int gt, j0, rb;
-        pass_tile<N1>(in, filt, 4, 2, t, gt, j0, rb, s0, s1);
-#pragma unroll
-        for (int p = 0; p < P::J; p++)
-#pragma unroll
-            for (int q = 0; q < P::R; q++) {
-                double *dst = coef + child_off + (long long)gt * stride + (j0 + p) * N2 + rb + q * P::RB;
-                double v = *dst;
-                v += s0[p][q];
-                v += s1[p][q];
-                *dst = v;
-            }
-    }
-}
-
-// The generation, top-down, bottom-up and product passes are latency-bound for
-// the few nodes of a launch: their workgroups have kPassThreads threads, each
-// forming a 2 x 2 register tile of a pass (the same per-output sum, over i in
-// increasing order, as the 4 x 4 tiles of mw_pass, so the same results).
-constexpr int kPassThreads = 1024;
-template <int N1> struct SmallTile {
-    static constexpr int N2 = N1 * N1, J = 2, R = 2, RB = N2 / R, JG = N1 / J, TILES = 8 * JG * RB;
-    static_assert(N1 % J == 0 && N2 % R == 0, "small pass tile shape");
-};
-template <int N1>
-__device__ __forceinline__ void small_tile(const double *in, const double *filt, int dir_base, int dim, int t, int &gt, int &j0, int &rb, double (&s0)[2][2],
-                                           double (&s1)[2][2]) {
-    using P = SmallTile<N1>;
-    constexpr int N2 = P::N2, N3 = N2 * N1, J = P::J, R = P::R, RB = P::RB;
-    gt = t / (P::JG * RB);
-    j0 = ((t / RB) % P::JG) * J;
-    rb = t % RB;
-    const int bit = 1 << dim;
-    const int ft0 = gt & ~bit, ft1 = gt | bit;
-    const double *F0 = filt + (size_t)(dir_base + 2 * ((gt >> dim) & 1) + 0) * N2 + N1 * j0;
-    const double *F1 = filt + (size_t)(dir_base + 2 * ((gt >> dim) & 1) + 1) * N2 + N1 * j0;
-#pragma unroll
-    for (int p = 0; p < J; p++)
-#pragma unroll
-        for (int q = 0; q < R; q++) {
-            s0[p][q] = 0.0;
-            s1[p][q] = 0.0;
-        }
-#pragma unroll 2
-    for (int i = 0; i < N1; i++) {
-        double x0[R], x1[R], f0[J], f1[J];
-#pragma unroll
-        for (int q = 0; q < R; q++) {
-            x0[q] = in[pad<N1>(ft0 * N3 + N1 * (rb + q * RB) + i)];
-            x1[q] = in[pad<N1>(ft1 * N3 + N1 * (rb + q * RB) + i)];
-        }
-#pragma unroll
-        for (int p = 0; p < J; p++) {
-            f0[p] = F0[N1 * p + i];
-            f1[p] = F1[N1 * p + i];
-        }
-#pragma unroll
-        for (int p = 0; p < J; p++)
-#pragma unroll
-            for (int q = 0; q < R; q++) {
-                s0[p][q] += x0[q] * f0[p];
-                s1[p][q] += x1[q] * f1[p];
-            }
-    }
-}
-template <int N1> __device__ __forceinline__ void small_pass(double *out, const double *in, const double *filt, int dir_base, int dim) {
-    using P = SmallTile<N1>;
-    constexpr int N2 = P::N2, N3 = N2 * N1;
-    for (int t = threadIdx.x; t < P::TILES; t += kPassThreads) {
-        double s0[2][2], s1[2][2];
-        int gt, j0, rb;
-        small_tile<N1>(in, filt, dir_base, dim, t, gt, j0, rb, s0, s1);
-#pragma unroll
-        for (int p = 0; p < 2; p++)
-#pragma unroll
-            for (int q = 0; q < 2; q++) out[pad<N1>(gt * N3 + (j0 + p) * N2 + rb + q * P::RB)] = s0[p][q] + s1[p][q];
-    }
-}
 // Component norms from the first kThreads threads' sums of squares ss[8],
 // written to nrm[0..8] (8 norms + square norm): lanes by a fixed tree, waves in
 // order.  Every thread of the workgroup must call.
@@ -360,15 +185,15 @@ __device__ inline void norms_of_sums(double (&ss)[8], double *nrm, double *red) 
     __syncthreads();
 }
 
-// Component norms of 8 blocks (PAD: c in the padded LDS layout).
-template <int N1, bool PAD = false> __device__ inline void block_norms(const double *c, double *nrm, double *red) {
+// Component norms of 8 blocks.
+template <int N1> __device__ inline void block_norms(const double *c, double *nrm, double *red) {
     constexpr int N3 = N1 * N1 * N1;
     double ss[8];
 #pragma unroll
     for (int t = 0; t < 8; t++) ss[t] = 0.0;
     if (threadIdx.x < kThreads)
         for (int o = threadIdx.x; o < 8 * N3; o += kThreads) {
-            const double v = c[PAD ? pad<N1>(o) : o];
+            const double v = c[o];
             ss[o / N3] += v * v;
         }
     norms_of_sums(ss, nrm, red);

@@ -1,120 +1,104 @@
 // Projection of a sum of Gaussians onto the nodes of one tree level
 // (ProjectionCalculator::calcNode, src/treebuilders/ProjectionCalculator.cpp:34-51).
 //
-// One 256-thread workgroup per node.  The function is sampled at the
+// One workgroup per node.  The function is sampled at the
 // Gauss-Legendre points of the node's 8 children (MWNode::getExpandedChildPts,
 // src/trees/MWNode.cpp:854-925): point (t, i0, i1, i2) sits at
 // sf_d 2^-(n+1) (x_{i_d} + 2 l_d + bit_d(t)).  A Gaussian is separable, so per
 // node and term the 3 x 2(k+1) one-dimensional factors exp(-alpha_d q^2) are
-// formed once in LDS and every point takes coef * e_x e_y e_z: 6(k+1) exp
+// formed once in LDS and every point takes (coef e_x e_y) e_z: 6(k+1) exp
 // evaluations per term instead of 8(k+1)^3.  Then the value -> coefficient
 // map in each direction (MWNode::cvTransform, :448-490), the scaling factor
 // sqrt(sf_x sf_y sf_z / 2^(3(n+1))), the compression to the node's scaling and
 // wavelet blocks (MWNode::mwTransform(Compression)) and the component norms.
-#include "device_common.h"
+#include "mw_passes.h"
 
 namespace mwgdev {
 
 namespace {
 
-constexpr int kTermsPerRound = 16; // Gaussian terms whose 1D factors share LDS at a time (LDS <= 80 KB at k = 7: two workgroups per CU)
+constexpr int kTermsPerRound = 16; // Gaussian terms whose 1D factors share LDS at a time
 
-// out(r, j) = sum_i in(i, r) V(i, j) for each of the 8 blocks (in viewed
-// N1 x N1^2, column-major; core::filter_pass), padded LDS layout.
-template <int N1> __device__ inline void vc_pass(double *out, const double *in, const double *V) {
-    constexpr int N2 = N1 * N1, N3 = N2 * N1;
-    for (int o = threadIdx.x; o < 8 * N3; o += kThreads) {
-        const int t = o / N3, e = o % N3;
-        const int r = e % N2, j = e / N2;
-        const double *x = in + pad<N1>(t * N3 + N1 * r);
-        const double *v = V + N1 * j;
-        double s = 0.0;
-#pragma unroll
-        for (int i = 0; i < N1; i++) s += x[i] * v[i];
-        out[pad<N1>(o)] = s;
-    }
-}
-
+// The value at a point is sum_g (c_g e_x e_y)(e_z): the points' values are a
+// product of a 4 N1^2 x terms matrix, formed as it is read, and a terms x 2 N1
+// matrix, in the tiles of a pass (mw_passes.h) and left as a pass in direction z
+// leaves them.  A pass takes the value -> coefficient map and the compression
+// filters of its direction, three passes in all.  Bound by the exponentials and the chain of
+// passes (points one by one on the vector units, maps and filters apart:
+// 142 -> 58 us a launch of order 7).
 template <int N1>
-__global__ __launch_bounds__(kThreads) void k_project(mwg_projection pj, const int *scale, const int *lv, const long long *off, double *coef,
-                                                      double *norms) {
-    constexpr int N2 = N1 * N1, N3 = N2 * N1, PT = (8 * N3 + kThreads - 1) / kThreads;
-    __shared__ double a[Lds<N1>::size], b[Lds<N1>::size];
-    __shared__ double fac1d[kTermsPerRound][3][2 * N1]; // exp(-alpha_d q^2) at the 2 N1 points of each direction
-    __shared__ double gcoef[kTermsPerRound];
-    __shared__ double red[8 * (kThreads / 64)];
-    __shared__ double sx[N1], svc[N2];
+__global__ __launch_bounds__(MwShape<N1>::THREADS, MwShape<N1>::OCC) void k_project(mwg_projection pj, const int *scale, const int *lv, const long long *off,
+                                                                  double *coef, double *norms) {
+    using P = MwShape<N1>;
+    constexpr int N2 = P::N2, W = 2 * N1, T = P::T, G = kTermsPerRound;
+    __shared__ double a[P::SIZE], b[P::SIZE];
+    // exp(-alpha_d q^2) at the 2 N1 points of each direction, in the buffer that
+    // the passes write first
+    static_assert(G * 3 * W <= P::SIZE, "factors fit a pass buffer");
+    double(*fac1d)[3][W] = reinterpret_cast<double(*)[3][W]>(b);
+    __shared__ double gcoef[G];
+    __shared__ double vcs[MwMap<N1>::STORE], red[8];
+    __shared__ double sx[N1];
     const int k = blockIdx.x;
     const int n = scale[k];
     const int l[3] = {lv[3 * k], lv[3 * k + 1], lv[3 * k + 2]};
     const double h = ldexp(1.0, -(n + 1));
-    for (int i = threadIdx.x; i < N1; i += kThreads) sx[i] = pj.nodes[i];
-    for (int i = threadIdx.x; i < N2; i += kThreads) svc[i] = pj.vcmap[i];
-    __syncthreads();
+    for (int i = threadIdx.x; i < N1; i += P::THREADS) sx[i] = pj.nodes[i];
+    MwMap<N1> vc;
+    if constexpr (MwMap<N1>::LDS) vc.load(pj.vcmap, vcs);
 
-    // function values: each thread owns points o = tid + 256 p
-    double val[PT];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = lane & 3, row = lane & 15, kk = lane >> 4;
+    double val[P::PER][T];
 #pragma unroll
-    for (int p = 0; p < PT; p++) val[p] = 0.0;
-    for (int g0 = 0; g0 < pj.ngauss; g0 += kTermsPerRound) {
-        const int ng = min(kTermsPerRound, pj.ngauss - g0);
-        __syncthreads(); // previous round's factors consumed
-        for (int q = threadIdx.x; q < ng * 3 * 2 * N1; q += kThreads) {
-            const int gi = q / (6 * N1), rest = q % (6 * N1), d = rest / (2 * N1), hi = rest % (2 * N1);
+    for (int q = 0; q < P::PER; q++)
+#pragma unroll
+        for (int J = 0; J < T; J++) val[q][J] = 0.0;
+    for (int g0 = 0; g0 < pj.ngauss; g0 += G) {
+        const int ng = min(G, pj.ngauss - g0), steps = (ng + 3) / 4;
+        __syncthreads(); // points staged; previous round's factors consumed
+        for (int p = threadIdx.x; p < 4 * steps * 3 * W; p += P::THREADS) {
+            const int gi = p / (3 * W), rest = p % (3 * W), d = rest / W, hi = rest % W;
             const int half = hi / N1, i = hi % N1;
-            const mwg_gauss &G = pj.gauss[g0 + gi];
-            const double base = sx[i] + 2.0 * (double)l[d];
-            const double r = pj.sf[d] * (h * (half ? base + 1.0 : base));
-            const double dq = r - G.pos[d];
-            fac1d[gi][d][hi] = exp(-(G.alpha[d] * dq * dq));
+            double e = 0.0; // terms past the last fill the step with zeros
+            if (gi < ng) {
+                const mwg_gauss &gs = pj.gauss[g0 + gi];
+                const double base = sx[i] + 2.0 * (double)l[d];
+                const double r = pj.sf[d] * (h * (half ? base + 1.0 : base));
+                const double dq = r - gs.pos[d];
+                e = exp(-(gs.alpha[d] * dq * dq));
+            }
+            fac1d[gi][d][hi] = e;
         }
-        for (int gi = threadIdx.x; gi < ng; gi += kThreads) gcoef[gi] = pj.gauss[g0 + gi].coef;
+        for (int gi = threadIdx.x; gi < 4 * steps; gi += P::THREADS) gcoef[gi] = gi < ng ? pj.gauss[g0 + gi].coef : 0.0;
         __syncthreads();
 #pragma unroll
-        for (int p = 0; p < PT; p++) {
-            const int o = threadIdx.x + kThreads * p;
-            if (o >= 8 * N3) break;
-            const int t = o / N3, e = o % N3;
-            const int ix = (t & 1) * N1 + e % N1, iy = ((t >> 1) & 1) * N1 + (e / N1) % N1, iz = ((t >> 2) & 1) * N1 + e / N2;
-            double v = val[p];
-            for (int gi = 0; gi < ng; gi++) v += gcoef[gi] * (fac1d[gi][0][ix] * fac1d[gi][1][iy] * fac1d[gi][2][iz]);
-            val[p] = v;
+        for (int q = 0; q < P::PER; q++) {
+            const int item = wave + P::WAVES * q;
+            if (P::ITEMS % P::WAVES != 0 && item >= P::ITEMS) break;
+            const int ra = 16 * item + row, c = ra / N2, e = ra - c * N2; // row: child bits (x, y), points (i_x, i_y)
+            const int ix = (c & 1) * N1 + e % N1, iy = (c >> 1) * N1 + e / N1;
+            for (int K = 0; K < steps; K++) {
+                const int gi = 4 * K + kk;
+                const double xy = gcoef[gi] * (fac1d[gi][0][ix] * fac1d[gi][1][iy]);
+#pragma unroll
+                for (int J = 0; J < T; J++) val[q][J] = __builtin_amdgcn_mfma_f64_4x4x4f64(fac1d[gi][2][4 * J + col], xy, val[q][J], 0, 0, 0);
+            }
         }
     }
-#pragma unroll
-    for (int p = 0; p < PT; p++) {
-        const int o = threadIdx.x + kThreads * p;
-        if (o < 8 * N3) a[pad<N1>(o)] = val[p];
-    }
-    __syncthreads();
-    // values -> coefficients, one direction per pass
-    vc_pass<N1>(b, a, svc);
-    __syncthreads();
-    vc_pass<N1>(a, b, svc);
-    __syncthreads();
-    vc_pass<N1>(b, a, svc);
-    __syncthreads();
     double sfp = pj.sf[0] * pj.sf[1] * pj.sf[2];
     if (sfp <= kMachineZero) sfp = 1.0;
     const double fac = sqrt(1.0 / (ldexp(1.0, 3 * (n + 1)) / sfp));
-    for (int o = threadIdx.x; o < 8 * N3; o += kThreads) b[pad<N1>(o)] *= fac;
+    if constexpr (!MwMap<N1>::LDS) vc.load(pj.vcmap, vcs);
+    mw_own<N1, 2>([&](int q, int J, int t, int j, int r) { a[P::at_out(t, j, r)] = fac * val[q][J]; });
     __syncthreads();
-    // children's scaling blocks -> the node's scaling and wavelet blocks
-    mw_pass<N1>(a, b, pj.filters, 0, 0); // filters read through the cache
-    __syncthreads();
-    mw_pass<N1>(b, a, pj.filters, 0, 1);
-    __syncthreads();
-    mw_pass<N1>(a, b, pj.filters, 0, 2);
-    __syncthreads();
-    double *dst = coef + off[k];
-    for (int o = threadIdx.x; o < 8 * N3; o += kThreads) dst[o] = a[pad<N1>(o)];
-    block_norms<N1, true>(a, norms + (size_t)k * 9, red);
+    mw_values_to_node<N1>(a, b, pj.filters, vc, coef + off[k], norms + (size_t)k * 9, red);
 }
 
 template <int N1> struct ProjectL {
     static mwg_status run(const mwg_projection *pj, const int *scale, const int *l, const long long *off, double *coef, double *norms, int count) {
         ProfileScope prof_(MWG_KERNEL_PROJECT);
-        hipLaunchKernelGGL(k_project<N1>, dim3(count), dim3(kThreads), 0, 0, *pj, scale, l, off, coef, norms);
+        hipLaunchKernelGGL(k_project<N1>, dim3(count), dim3(MwShape<N1>::THREADS), 0, 0, *pj, scale, l, off, coef, norms);
         MWG_LAUNCHED();
         return MWG_OK;
     }

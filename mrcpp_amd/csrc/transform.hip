@@ -1,62 +1,52 @@
 // Multiwavelet transforms on the device: generated band nodes, top-down
-// reconstruction, bottom-up compression and component norms.  One 256-thread
-// workgroup per node; the 8 blocks of a node are staged in LDS.
-#include "device_common.h"
+// reconstruction, bottom-up compression and component norms.  One workgroup per
+// node; a node's values go from HBM into the first pass's operands, through LDS
+// twice, and from the last pass's results back (passes on the vector units with
+// the node staged in LDS: compression 10.3 -> 8.4 us a launch at order 7, 24 ->
+// 13 at order 9; generation 16 -> 9 at order 9).  A launch's few nodes leave most
+// of that to its latency: the loads, two barriers and the stores of one node.
+#include "mw_passes.h"
 
 namespace mwgdev {
 
 namespace {
 
-template <int N1>
-__device__ __forceinline__ void small_pass_add_children(double *coef, long long child_off, long long stride, const double *in, const double *filt) {
-    using P = SmallTile<N1>;
-    constexpr int N2 = P::N2;
-    for (int t = threadIdx.x; t < P::TILES; t += kPassThreads) {
-        double s0[2][2], s1[2][2];
-        int gt, j0, rb;
-        small_tile<N1>(in, filt, 4, 2, t, gt, j0, rb, s0, s1);
-#pragma unroll
-        for (int p = 0; p < 2; p++)
-#pragma unroll
-            for (int q = 0; q < 2; q++) {
-                double *dst = coef + child_off + (long long)gt * stride + (j0 + p) * N2 + rb + q * P::RB;
-                double v = *dst;
-                v += s0[p][q];
-                v += s1[p][q];
-                *dst = v;
-            }
-    }
-}
-
-// The scaling block of child c of node pid (staged filters sfl; a, b, red:
-// LDS of the workgroup), written at offs[k] (recorded in the tree) or at the
+// The scaling block of child c of node pid (a, b, red: LDS of the workgroup),
+// written at offs[k] (recorded in the tree) or at the
 // node's own offset, and its norms.
 template <int N1>
-__device__ __forceinline__ void generate_node(const mwg_ftree &f, const double *sfl, int k, int id, int pid, int c, const long long *offs,
+__device__ __forceinline__ void generate_node(const mwg_ftree &f, const double *filt, int k, int id, int pid, int c, const long long *offs,
                                               long long *coef_off_w, unsigned char *is_gen_w, double *a, double *b, double *red) {
-    constexpr int N3 = N1 * N1 * N1;
+    using P = MwShape<N1>;
+    constexpr int N3 = P::N3;
     const double *src = f.coef + f.coef_off[pid];
-    const int nblk = f.is_gen[pid] ? 1 : 8; // generated parents carry the scaling block only
-    for (int o = threadIdx.x; o < 8 * N3; o += kPassThreads) a[pad<N1>(o)] = (o < nblk * N3) ? src[o] : 0.0;
+    const bool gen = f.is_gen[pid]; // generated parents carry the scaling block only
+    MwMatrix<N1> M;
+    M.filters(filt, 4);
+    mw_pass<N1, 0>(
+        M, [&](int t, int r, int i) { return gen && t != 0 ? 0.0 : src[t * N3 + N1 * r + i]; },
+        [&](int, int, int t, int j, int r, double v) { a[P::at_out(t, j, r)] = v; });
     __syncthreads();
-    small_pass<N1>(b, a, sfl, 4, 0);
+    mw_pass_lds<N1, 1>(b, a, M);
     __syncthreads();
-    small_pass<N1>(a, b, sfl, 4, 1);
-    __syncthreads();
-    small_pass<N1>(b, a, sfl, 4, 2);
+    mw_pass<N1, 2>(
+        M, [&](int t, int r, int i) { return b[P::at(t, r, i)]; },
+        [&](int, int, int t, int j, int r, double v) {
+            if (t == c) a[P::at_out(0, j, r)] = v;
+        });
     __syncthreads();
     double *dst = f.coef + (offs ? offs[k] : f.coef_off[id]);
     if (offs && threadIdx.x == 0) {
         coef_off_w[id] = offs[k];
         is_gen_w[id] = 1;
     }
-    for (int e = threadIdx.x; e < N3; e += kPassThreads) dst[e] = b[pad<N1>(c * N3 + e)];
+    for (int e = threadIdx.x; e < N3; e += P::THREADS) dst[e] = a[P::at_elem(0, e)];
     // the norm summed by the first kThreads threads in their order (the
     // order of the band screen's other norms)
     if (threadIdx.x < kThreads) {
         double ss = 0.0;
         for (int e = threadIdx.x; e < N3; e += kThreads) {
-            const double v = b[pad<N1>(c * N3 + e)];
+            const double v = a[P::at_elem(0, e)];
             ss += v * v;
         }
         for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off);
@@ -79,67 +69,68 @@ __device__ __forceinline__ void generate_node(const mwg_ftree &f, const double *
 // With offs given, the node is also recorded in the mirror: coef_off_w[id] =
 // offs[k] (where its block goes) and is_gen_w[id] = 1.
 template <int N1>
-__global__ __launch_bounds__(kPassThreads) void k_generate(mwg_ftree f, const double *filt, const int *ids, const int *parent, const int *child,
+__global__ __launch_bounds__(MwShape<N1>::THREADS, MwShape<N1>::OCC) void k_generate(mwg_ftree f, const double *filt, const int *ids, const int *parent, const int *child,
                                                            const long long *offs, long long *coef_off_w, unsigned char *is_gen_w) {
-    __shared__ double a[Lds<N1>::size], b[Lds<N1>::size];
-    __shared__ double red[8 * (kThreads / 64)];
-    __shared__ double sfl[8 * N1 * N1];
-    for (int i = threadIdx.x; i < 8 * N1 * N1; i += kPassThreads) sfl[i] = filt[i];
+    __shared__ double a[MwShape<N1>::SIZE], b[MwShape<N1>::SIZE];
+    __shared__ double red[kThreads / 64];
     const int k = blockIdx.x;
-    generate_node<N1>(f, sfl, k, ids[k], parent[k], child[k], offs, coef_off_w, is_gen_w, a, b, red);
+    generate_node<N1>(f, filt, k, ids[k], parent[k], child[k], offs, coef_off_w, is_gen_w, a, b, red);
 }
 
 // The same for nodes of several trees: node k in trees[tree_of[k]].
 template <int N1>
-__global__ __launch_bounds__(kPassThreads) void k_generate_multi(const mwg_gen_tree *trees, const double *filt, const int *tree_of, const int *ids,
+__global__ __launch_bounds__(MwShape<N1>::THREADS, MwShape<N1>::OCC) void k_generate_multi(const mwg_gen_tree *trees, const double *filt, const int *tree_of, const int *ids,
                                                                  const int *parent, const int *child, const long long *offs) {
-    __shared__ double a[Lds<N1>::size], b[Lds<N1>::size];
-    __shared__ double red[8 * (kThreads / 64)];
-    __shared__ double sfl[8 * N1 * N1];
-    for (int i = threadIdx.x; i < 8 * N1 * N1; i += kPassThreads) sfl[i] = filt[i];
+    __shared__ double a[MwShape<N1>::SIZE], b[MwShape<N1>::SIZE];
+    __shared__ double red[kThreads / 64];
     const int k = blockIdx.x;
     const mwg_gen_tree &t = trees[tree_of[k]];
-    generate_node<N1>(t.f, sfl, k, ids[k], parent[k], child[k], offs, t.coef_off_w, t.is_gen_w, a, b, red);
+    generate_node<N1>(t.f, filt, k, ids[k], parent[k], child[k], offs, t.coef_off_w, t.is_gen_w, a, b, red);
 }
 
 template <int N1>
-__global__ __launch_bounds__(kPassThreads) void k_reconstruct_add(const double *filt, double *coef, const long long *poff, const long long *coff,
-                                                                  long long stride) {
-    constexpr int N3 = N1 * N1 * N1;
-    __shared__ double a[Lds<N1>::size], b[Lds<N1>::size];
-    __shared__ double sfl[8 * N1 * N1];
-    for (int i = threadIdx.x; i < 8 * N1 * N1; i += kPassThreads) sfl[i] = filt[i];
+__global__ __launch_bounds__(MwShape<N1>::THREADS, MwShape<N1>::OCC) void k_reconstruct_add(const double *filt, double *coef, const long long *poff,
+                                                                                            const long long *coff, long long stride) {
+    using P = MwShape<N1>;
+    __shared__ double a[P::SIZE], b[P::SIZE];
     const int k = blockIdx.x;
     const double *src = coef + poff[k];
-    for (int o = threadIdx.x; o < 8 * N3; o += kPassThreads) a[pad<N1>(o)] = src[o];
+    double *dst = coef + coff[k];
+    MwMatrix<N1> M;
+    M.filters(filt, 4);
+    mw_pass<N1, 0>(
+        M, [&](int t, int r, int i) { return src[t * P::N3 + N1 * r + i]; },
+        [&](int, int, int t, int j, int r, double v) { a[P::at_out(t, j, r)] = v; });
+    // the children's values as they are, in flight during the second pass
+    double old[P::PER][P::T];
+    mw_own<N1, 2>([&](int q, int J, int t, int j, int r) { old[q][J] = dst[t * stride + j * P::N2 + r]; });
     __syncthreads();
-    small_pass<N1>(b, a, sfl, 4, 0);
+    mw_pass_lds<N1, 1>(b, a, M);
     __syncthreads();
-    small_pass<N1>(a, b, sfl, 4, 1);
-    __syncthreads();
-    small_pass_add_children<N1>(coef, coff[k], stride, a, sfl);
+    mw_pass<N1, 2>(
+        M, [&](int t, int r, int i) { return b[P::at(t, r, i)]; },
+        [&](int q, int J, int t, int j, int r, double v) { dst[t * stride + j * P::N2 + r] = old[q][J] + v; });
 }
 
 template <int N1>
-__global__ __launch_bounds__(kPassThreads) void k_compress(const double *filt, double *coef, const long long *poff, const long long *coff, long long stride) {
-    constexpr int N3 = N1 * N1 * N1;
-    __shared__ double a[Lds<N1>::size], b[Lds<N1>::size];
-    __shared__ double sfl[4 * N1 * N1];
-    for (int i = threadIdx.x; i < 4 * N1 * N1; i += kPassThreads) sfl[i] = filt[i];
+__global__ __launch_bounds__(MwShape<N1>::THREADS, MwShape<N1>::OCC) void k_compress(const double *filt, double *coef, const long long *poff,
+                                                                                     const long long *coff, long long stride) {
+    using P = MwShape<N1>;
+    __shared__ double a[P::SIZE], b[P::SIZE];
     const int k = blockIdx.x;
-    for (int o = threadIdx.x; o < 8 * N3; o += kPassThreads) {
-        const int t = o / N3, e = o % N3;
-        a[pad<N1>(o)] = coef[coff[k] + (long long)t * stride + e];
-    }
-    __syncthreads();
-    small_pass<N1>(b, a, sfl, 0, 0);
-    __syncthreads();
-    small_pass<N1>(a, b, sfl, 0, 1);
-    __syncthreads();
-    small_pass<N1>(b, a, sfl, 0, 2);
-    __syncthreads();
+    const double *src = coef + coff[k];
     double *dst = coef + poff[k];
-    for (int o = threadIdx.x; o < 8 * N3; o += kPassThreads) dst[o] = b[pad<N1>(o)];
+    MwMatrix<N1> M;
+    M.filters(filt, 0);
+    mw_pass<N1, 0>(
+        M, [&](int t, int r, int i) { return src[t * stride + N1 * r + i]; },
+        [&](int, int, int t, int j, int r, double v) { a[P::at_out(t, j, r)] = v; });
+    __syncthreads();
+    mw_pass_lds<N1, 1>(b, a, M);
+    __syncthreads();
+    mw_pass<N1, 2>(
+        M, [&](int t, int r, int i) { return b[P::at(t, r, i)]; },
+        [&](int, int, int t, int j, int r, double v) { dst[t * P::N3 + j * P::N2 + r] = v; });
 }
 
 template <int N1> __global__ __launch_bounds__(kThreads) void k_node_norms(const double *coef, const long long *off, double *norms) {
@@ -152,7 +143,7 @@ template <int N1> struct GenerateL {
     static mwg_status run(const mwg_ftree *f, const double *filt, const int *ids, const int *par, const int *ch, int count, const long long *offs,
                           long long *coef_off_w, unsigned char *is_gen_w) {
         ProfileScope prof_(MWG_KERNEL_GENERATE);
-        hipLaunchKernelGGL(k_generate<N1>, dim3(count), dim3(kPassThreads), 0, 0, *f, filt, ids, par, ch, offs, coef_off_w, is_gen_w);
+        hipLaunchKernelGGL(k_generate<N1>, dim3(count), dim3(MwShape<N1>::THREADS), 0, 0, *f, filt, ids, par, ch, offs, coef_off_w, is_gen_w);
         MWG_LAUNCHED();
         return MWG_OK;
     }
@@ -161,7 +152,7 @@ template <int N1> struct GenerateMultiL {
     static mwg_status run(const mwg_gen_tree *trees, const double *filt, const int *tree_of, const int *ids, const int *par, const int *ch,
                           const long long *offs, int count) {
         ProfileScope prof_(MWG_KERNEL_GENERATE);
-        hipLaunchKernelGGL(k_generate_multi<N1>, dim3(count), dim3(kPassThreads), 0, 0, trees, filt, tree_of, ids, par, ch, offs);
+        hipLaunchKernelGGL(k_generate_multi<N1>, dim3(count), dim3(MwShape<N1>::THREADS), 0, 0, trees, filt, tree_of, ids, par, ch, offs);
         MWG_LAUNCHED();
         return MWG_OK;
     }
@@ -169,7 +160,7 @@ template <int N1> struct GenerateMultiL {
 template <int N1> struct ReconL {
     static mwg_status run(const double *filt, double *coef, const long long *po, const long long *co, int count, long long stride) {
         ProfileScope prof_(MWG_KERNEL_RECONSTRUCT);
-        hipLaunchKernelGGL(k_reconstruct_add<N1>, dim3(count), dim3(kPassThreads), 0, 0, filt, coef, po, co, stride);
+        hipLaunchKernelGGL(k_reconstruct_add<N1>, dim3(count), dim3(MwShape<N1>::THREADS), 0, 0, filt, coef, po, co, stride);
         MWG_LAUNCHED();
         return MWG_OK;
     }
@@ -177,7 +168,7 @@ template <int N1> struct ReconL {
 template <int N1> struct CompressL {
     static mwg_status run(const double *filt, double *coef, const long long *po, const long long *co, int count, long long stride) {
         ProfileScope prof_(MWG_KERNEL_COMPRESS);
-        hipLaunchKernelGGL(k_compress<N1>, dim3(count), dim3(kPassThreads), 0, 0, filt, coef, po, co, stride);
+        hipLaunchKernelGGL(k_compress<N1>, dim3(count), dim3(MwShape<N1>::THREADS), 0, 0, filt, coef, po, co, stride);
         MWG_LAUNCHED();
         return MWG_OK;
     }

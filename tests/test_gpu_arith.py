@@ -5,8 +5,8 @@ tests/test_arith_oracle.py pins to closed forms.
 
 Inputs are projected on the host so both sides start from bit-identical trees.
 Bar: identical node sets; coefficients within 1e-14 relative L2 of the
-oracle's (both compute the nodes without fused multiply-adds in the same order;
-the device's norm sums and bottom-up transform round differently).
+oracle's (sums without fused multiply-adds in the same order; the device's
+products, norm sums and bottom-up transform round differently).
 """
 import math
 import sys
