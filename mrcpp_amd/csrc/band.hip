@@ -253,18 +253,16 @@ __device__ inline int units_group_size(int gmin, int total, int slots, int T) {
 // unit and the first partial slot of every node.  With all_slots (the wave
 // kernels) a node of several units has a slot for each, else for each but the
 // first, which writes the node itself; the flag marks the units without one.
-__global__ __launch_bounds__(256) void k_unit_count(int L, mwg_pairs pr, int npairs, const int *gstart, int gmin, int slots, bool all_slots, long long *packed, int *counter,
-                                                    const mwg_segment *segs, const int *node_seg, const int *papp, const double *pmg, double *g_margin) {
-    const int g = blockIdx.x * 256 + threadIdx.x;
-    if (g == 0) *counter = 0;
+// The node has np pairs from gf on, with T groups and app applied tuples, total
+// groups in the level.  Every thread of a wave calls, with node g live or not; the
+// node's counters and margins are added up on the way.
+__device__ __forceinline__ long long node_units(int g, bool live, int gf, int np, int T, unsigned long long app, int total, int gmin, int slots,
+                                                bool all_slots, const mwg_segment *segs, const int *node_seg, const double *pmg, double *g_margin) {
     // applied tuples and candidate pairs of the node's pairs, added to its
     // segment's counters: one atomic per wave when the wave's nodes share a
     // segment (lane 0 holds the wave's first node)
-    const bool live = g < L;
-    const int gf = live ? pr.g_first[g] : 0, np = live ? pr.g_npairs[g] : 0;
     const int s = live ? node_seg[g] : -1;
-    unsigned long long app = 0, npl = (unsigned long long)np;
-    for (int q = gf; q < gf + np; q++) app += (unsigned)papp[q];
+    unsigned long long npl = (unsigned long long)np;
     const int s0 = __shfl(s, 0);
     if (__all(!live || s == s0)) {
         for (int off = 32; off > 0; off >>= 1) {
@@ -279,7 +277,7 @@ __global__ __launch_bounds__(256) void k_unit_count(int L, mwg_pairs pr, int npa
         if (app) atomicAdd(segs[s].counters, app);
         if (np) atomicAdd(segs[s].counters + 1, npl);
     }
-    if (!live) return;
+    if (!live) return 0;
     if (g_margin) { // the node's screening margins, its pairs in order
         double m[MWG_MARGINS];
 #pragma unroll
@@ -290,10 +288,67 @@ __global__ __launch_bounds__(256) void k_unit_count(int L, mwg_pairs pr, int npa
 #pragma unroll
         for (int j = 0; j < MWG_MARGINS; j++) g_margin[MWG_MARGINS * (size_t)g + j] = m[j];
     }
-    const int T = gstart[gf + np] - gstart[gf];
-    const int G = units_group_size(gmin, gstart[npairs], slots, T);
+    const int G = units_group_size(gmin, total, slots, T);
     const int nu = (T + G - 1) / G;
-    packed[g] = (long long)nu + ((long long)(all_slots ? nu == 1 : nu > 0) << 32);
+    return (long long)nu + ((long long)(all_slots ? nu == 1 : nu > 0) << 32);
+}
+
+__global__ __launch_bounds__(256) void k_unit_count(int L, mwg_pairs pr, int npairs, const int *gstart, int gmin, int slots, bool all_slots, long long *packed, int *counter,
+                                                    const mwg_segment *segs, const int *node_seg, const int *papp, const double *pmg, double *g_margin) {
+    const int g = blockIdx.x * 256 + threadIdx.x;
+    if (g == 0) *counter = 0;
+    const bool live = g < L;
+    const int gf = live ? pr.g_first[g] : 0, np = live ? pr.g_npairs[g] : 0;
+    unsigned long long app = 0;
+    for (int q = gf; q < gf + np; q++) app += (unsigned)papp[q];
+    const long long v = node_units(g, live, gf, np, live ? gstart[gf + np] - gstart[gf] : 0, app, gstart[npairs], gmin, slots, all_slots, segs, node_seg,
+                                   pmg, g_margin);
+    if (live) packed[g] = v;
+}
+
+// The plan of a level of at most kPlanPairs pairs and kPlanNodes nodes in one
+// workgroup: groups per pair (gstart) and units per node (packed) become prefix
+// sums, the applied tuples of a node a difference of them, all in LDS, in one
+// launch where longer levels take three (scan, k_unit_count, scan).  Plans and
+// screening of an application: 184 -> 162 us at order 5, 397 -> 360 at order 7.
+// The bounds are what one workgroup's LDS and threads hold; at them the work is
+// spread over more workgroups anyway.
+constexpr int kPlanPairs = 16384, kPlanNodes = 1024;
+__global__ __launch_bounds__(kPlanNodes) void k_unit_plan(int L, mwg_pairs pr, int npairs, int *gstart, int gmin, int slots, bool all_slots, long long *packed, int *counter,
+                                                          const mwg_segment *segs, const int *node_seg, const int *papp, const double *pmg,
+                                                          double *g_margin) {
+    // groups of a pair, applied tuples in the upper half; then before a pair
+    __shared__ unsigned long long gs[kPlanPairs + kPlanPairs / 16 + 1];
+    __shared__ unsigned long long ti[kPlanNodes / 64];
+    __shared__ long long tl[kPlanNodes / 64];
+    const auto at = [](int q) { return q + (q >> 4); }; // threads' runs start on different banks
+    const int tid = threadIdx.x;
+    const bool live = tid < L;
+    const int gf = live ? pr.g_first[tid] : 0, np = live ? pr.g_npairs[tid] : 0;
+    if (tid == 0) *counter = 0;
+    for (int q = tid; q < npairs; q += kPlanNodes) gs[at(q)] = (unsigned long long)(unsigned)gstart[q] | (unsigned long long)(unsigned)papp[q] << 32;
+    __syncthreads();
+    const int c = (npairs + kPlanNodes - 1) / kPlanNodes;
+    const int a = min(npairs, tid * c), b = min(npairs, a + c);
+    unsigned long long s = 0;
+    for (int q = a; q < b; q++) s += gs[at(q)];
+    unsigned long long before;
+    const unsigned long long total = block_exclusive_scan<unsigned long long, kPlanNodes>(s, ti, before);
+    for (int q = a; q < b; q++) {
+        const unsigned long long n = gs[at(q)];
+        gs[at(q)] = before;
+        before += n;
+    }
+    if (tid == 0) gs[at(npairs)] = total;
+    __syncthreads();
+    for (int q = tid; q <= npairs; q += kPlanNodes) gstart[q] = (int)(unsigned)gs[at(q)];
+    const unsigned long long mine = gs[at(gf + np)] - gs[at(gf)];
+    const long long v = node_units(tid, live, gf, np, (int)(unsigned)mine, mine >> 32, (int)(unsigned)total, gmin, slots, all_slots, segs, node_seg, pmg,
+                                   g_margin);
+    long long units;
+    const long long all = block_exclusive_scan<long long, kPlanNodes>(v, tl, units);
+    if (live) packed[tid] = units;
+    if (tid == 0) packed[L] = all;
 }
 
 __device__ inline int unit_first(long long v) { return (int)(v & 0xffffffffll); }
@@ -1211,13 +1266,19 @@ template <int N1> struct BandL {
             hipLaunchKernelGGL(k_group_screen, dim3(npairs), dim3(64 * kScreenWaves), 0, 0, dev.segs, dev.node_seg, lvl->l, lvl->node_thr, *pr,
                                w.codes.as<unsigned>(), stride, gstart, w.pdl.as<int4>(), w.pfo.as<long long>(), w.papp.as<int>(), mg);
             MWG_LAUNCHED();
-            mwg_status s = scan_exclusive(gstart, gstart, npairs);
-            if (s != MWG_OK) return s;
-            hipLaunchKernelGGL(k_unit_count, dim3((L + 255) / 256), dim3(256), 0, 0, L, *pr, npairs, gstart, g_unit_groups, slots, waves, uscan, w.counter.as<int>(),
-                               dev.segs, dev.node_seg, w.papp.as<int>(), mg.pair, lvl->g_margin);
-            MWG_LAUNCHED();
-            s = scan_exclusive(uscan, uscan, L);
-            if (s != MWG_OK) return s;
+            if (npairs <= kPlanPairs && L <= kPlanNodes) {
+                hipLaunchKernelGGL(k_unit_plan, dim3(1), dim3(kPlanNodes), 0, 0, L, *pr, npairs, gstart, g_unit_groups, slots, waves, uscan,
+                                   w.counter.as<int>(), dev.segs, dev.node_seg, w.papp.as<int>(), mg.pair, lvl->g_margin);
+                MWG_LAUNCHED();
+            } else {
+                mwg_status s = scan_exclusive(gstart, gstart, npairs);
+                if (s != MWG_OK) return s;
+                hipLaunchKernelGGL(k_unit_count, dim3((L + 255) / 256), dim3(256), 0, 0, L, *pr, npairs, gstart, g_unit_groups, slots, waves, uscan,
+                                   w.counter.as<int>(), dev.segs, dev.node_seg, w.papp.as<int>(), mg.pair, lvl->g_margin);
+                MWG_LAUNCHED();
+                s = scan_exclusive(uscan, uscan, L);
+                if (s != MWG_OK) return s;
+            }
             hipLaunchKernelGGL(k_unit_write, dim3(npairs), dim3(64), 0, 0, npairs, *pr, gstart, uscan, g_unit_groups, slots, w.units.as<int4>(), w.codes.as<unsigned>(),
                                stride, mfma ? w.grec.as<int2>() : nullptr, wr);
             MWG_LAUNCHED();
@@ -1239,6 +1300,14 @@ template <int N1> struct BandL {
         {
             ProfileScope prof_(MWG_KERNEL_REDUCE);
             const dim3 rgrid(L, (8 * N3 + 255) / 256);
+            if constexpr (N1 == 4) {
+                if (waves) {
+                    hipLaunchKernelGGL(k_reduce_norms, dim3(L), dim3(512), 0, 0, dev.segs, dev.node_seg, lvl->g_off, uscan, w.partial.as<double>(),
+                                       lvl->g_norms);
+                    MWG_LAUNCHED();
+                    return MWG_OK;
+                }
+            }
             if (!waves)
                 hipLaunchKernelGGL(k_reduce_units<N1>, rgrid, dim3(256), 0, 0, dev.segs, dev.node_seg, lvl->g_off, uscan, w.partial.as<double>());
             else if (precision == MWG_PREC_FP64)

@@ -621,8 +621,23 @@ template <int N1> __global__ __launch_bounds__(64, WaveLds<N1>::WAVES) void k_ba
     }
 }
 
-// Slots of the nodes of more than one unit added in unit order; a thread per
-// value of the slots' layout, their loads issued 8 at a time.
+// Slots of the nodes of more than one unit added in unit order, eight slots'
+// loads in flight: v0 + v1 + ... of one value, src[j stride] that of slot j.
+__device__ __forceinline__ double slot_sum(const double *src, int nu, size_t stride) {
+    double acc = src[0];
+    int j = 1;
+    for (; j + 8 <= nu; j += 8) {
+        double t[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) t[q] = src[(size_t)(j + q) * stride];
+#pragma unroll
+        for (int q = 0; q < 8; q++) acc += t[q];
+    }
+    for (; j < nu; j++) acc += src[(size_t)j * stride];
+    return acc;
+}
+
+// A thread per value of the slots' layout.
 template <int N1, int PREC>
 __global__ __launch_bounds__(256) void k_reduce_waves(const mwg_segment *segs, const int *node_seg, const long long *g_off, const long long *uscan,
                                                       const double *partial) {
@@ -634,24 +649,36 @@ __global__ __launch_bounds__(256) void k_reduce_waves(const mwg_segment *segs, c
     const int nu = unit_first(uscan[g + 1]) - Ug;
     if (nu == 1 || e >= 8 * W::N3) return; // a single unit wrote the node already
     double *dst = ro(segs)[ro(node_seg)[g]].g_coef + g_off[g];
-    const int lane = e & 63, row = e >> 6;
-    const int o = WaveMap<N1, PREC>::out(row / W::VALS, row % W::VALS, lane);
-    if (nu == 0) {
-        dst[o] = 0.0;
-        return;
+    const int o = WaveMap<N1, PREC>::out((e >> 6) / W::VALS, (e >> 6) % W::VALS, e & 63);
+    dst[o] = nu == 0 ? 0.0 : slot_sum(partial + (size_t)(Ug - flagged_before(v)) * 8 * W::N3 + e, nu, 8 * W::N3);
+}
+
+// The same at order 3 with the component norms (block_norms' order) in one
+// launch, a workgroup per node and a thread per value: its levels are short, and a
+// launch costs more than the 512 values (two launches: 56 us an application,
+// one: 47).  At the higher orders a workgroup per node leaves the slots' loads
+// too few workgroups (order 7: 289 -> 376 us an application, order 9: 206 -> 381).
+__global__ __launch_bounds__(512) void k_reduce_norms(const mwg_segment *segs, const int *node_seg, const long long *g_off, const long long *uscan,
+                                                      const double *partial, double *g_norms) {
+    using W = WaveShape<4>;
+    static_assert(8 * W::N3 == 512, "a thread per value");
+    __shared__ double c[512];
+    __shared__ double red[8 * (kThreads / 64)];
+    const int g = blockIdx.x, e = threadIdx.x;
+    const long long v = uscan[g];
+    const int Ug = unit_first(v);
+    const int nu = unit_first(uscan[g + 1]) - Ug;
+    double *dst = ro(segs)[ro(node_seg)[g]].g_coef + g_off[g];
+    if (nu == 1) {
+        c[e] = dst[e];
+    } else {
+        const int o = WaveMap<4, MWG_PREC_FP64>::out((e >> 6) / W::VALS, (e >> 6) % W::VALS, e & 63);
+        const double x = nu == 0 ? 0.0 : slot_sum(partial + (size_t)(Ug - flagged_before(v)) * 512 + e, nu, 512);
+        c[o] = x;
+        dst[o] = x;
     }
-    const double *src = partial + (size_t)(Ug - flagged_before(v)) * 8 * W::N3 + e;
-    double acc = src[0];
-    int j = 1;
-    for (; j + 8 <= nu; j += 8) {
-        double t[8];
-#pragma unroll
-        for (int q = 0; q < 8; q++) t[q] = src[(size_t)(j + q) * 8 * W::N3];
-#pragma unroll
-        for (int q = 0; q < 8; q++) acc += t[q];
-    }
-    for (; j < nu; j++) acc += src[(size_t)j * 8 * W::N3];
-    dst[o] = acc;
+    __syncthreads();
+    block_norms<4>(c, g_norms + (size_t)g * 9, red);
 }
 
 } // namespace
