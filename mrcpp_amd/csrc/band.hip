@@ -52,6 +52,12 @@ __device__ inline bool code_fresh(unsigned c) { return (c >> 31) != 0u; }
 
 // ---------------------------------------------------------------------------
 // 1. exact screening, two waves per pair
+//
+// Bound by the latency of a pair's chain of lookups, so by the waves in
+// flight: without the margins' sums a thread needs 95 registers (five waves per
+// SIMD; 154 and three with them), and both waves emit, every chunk of 64 terms
+// knowing its place from the chunks' counts (one wave emitted alone before).  The
+// order-7 Helmholtz application of 32 Gaussians: 1.42 -> 1.03 ms.
 // ---------------------------------------------------------------------------
 constexpr int kScreenWaves = 2; // waves per pair: wave v tests terms 64 v, 64 v + 1, ... (stride 128)
 
@@ -62,10 +68,12 @@ struct MarginSpec {
     double *pair; // [pair][MWG_MARGINS], nullptr: margins not computed
 };
 
-__global__ __launch_bounds__(64 * kScreenWaves) void k_group_screen(const mwg_segment *segs, const int *node_seg, const int *l, const double *node_thr,
+template <bool MARGINS>
+__global__ __launch_bounds__(64 * kScreenWaves, MARGINS ? 3 : 5) void k_group_screen(const mwg_segment *segs, const int *node_seg, const int *l, const double *node_thr,
                                                                    mwg_pairs pr, unsigned *codes, int stride, int *gcount, int4 *pdl, long long *pfo,
                                                                    int *papp, MarginSpec mg) {
     __shared__ unsigned char smask[8 * kMaxTerms];
+    __shared__ unsigned char s_cnt[8][(kMaxTerms + 63) / 64]; // groups of (f component, 64 terms)
     __shared__ unsigned s_napp[kScreenWaves];
     __shared__ double s_mg[kScreenWaves][MWG_MARGINS];
     __shared__ int sb40[kMaxTerms]; // band block index of each term (first matrix / 4 + width)
@@ -82,7 +90,7 @@ __global__ __launch_bounds__(64 * kScreenWaves) void k_group_screen(const mwg_se
             gcount[p] = 0;
             papp[p] = 0;
         }
-        if (mg.pair && threadIdx.x < MWG_MARGINS) mg.pair[MWG_MARGINS * (size_t)p + threadIdx.x] = 0.0;
+        if (MARGINS && threadIdx.x < MWG_MARGINS) mg.pair[MWG_MARGINS * (size_t)p + threadIdx.x] = 0.0;
         return;
     }
     double mg_thr[MWG_MARGINS], mg_sum[MWG_MARGINS];
@@ -177,7 +185,7 @@ __global__ __launch_bounds__(64 * kScreenWaves) void k_group_screen(const mwg_se
                     const double val = onorm * fthr;
                     if (val > g_thr) {
                         m |= 1u << gt;
-                        if (mg.pair) {
+                        if (MARGINS) {
                             const double c = onorm * fn[ft];
 #pragma unroll
                             for (int j = 0; j < MWG_MARGINS; j++)
@@ -192,12 +200,17 @@ __global__ __launch_bounds__(64 * kScreenWaves) void k_group_screen(const mwg_se
         if (i < M)
 #pragma unroll
             for (int ft = 0; ft < 8; ft++) smask[ft * M + i] = (unsigned char)m8[ft];
+#pragma unroll
+        for (int ft = 0; ft < 8; ft++) {
+            const int n = __popcll(__ballot(m8[ft] != 0));
+            if (lane == 0) s_cnt[ft][c0 / 64] = (unsigned char)n;
+        }
     }
     // applied tuples of the pair (added to the segment's counter per output
     // node by k_unit_count: one atomic per node instead of one per wave)
     for (int off = 32; off > 0; off >>= 1) napp += __shfl_xor(napp, off);
     if (lane == 0) s_napp[wv] = napp;
-    if (mg.pair) { // fixed-order tree over lanes, then waves in order
+    if (MARGINS) { // fixed-order tree over lanes, then waves in order
 #pragma unroll
         for (int j = 0; j < MWG_MARGINS; j++) {
             double x = mg_sum[j];
@@ -206,36 +219,36 @@ __global__ __launch_bounds__(64 * kScreenWaves) void k_group_screen(const mwg_se
         }
     }
     __syncthreads();
-    if (wv != 0) return;
-    if (lane == 0) {
+    if (threadIdx.x == 0) {
         unsigned tot = 0;
         for (int v = 0; v < kScreenWaves; v++) tot += s_napp[v];
         papp[p] = (int)tot;
     }
-    if (mg.pair && lane < MWG_MARGINS) {
+    if (MARGINS && threadIdx.x < MWG_MARGINS) {
         double x = 0.0;
-        for (int v = 0; v < kScreenWaves; v++) x += s_mg[v][lane];
-        mg.pair[MWG_MARGINS * (size_t)p + lane] = x;
+        for (int v = 0; v < kScreenWaves; v++) x += s_mg[v][threadIdx.x];
+        mg.pair[MWG_MARGINS * (size_t)p + threadIdx.x] = x;
     }
-    // emit ft-major, terms ascending
+    // emit ft-major, terms ascending: the chunks' counts give each its place, and
+    // a wave emits the chunks it tested
     int base = 0;
     unsigned *dst = codes + (size_t)p * stride;
     const unsigned long long below = (1ull << lane) - 1ull;
     for (int ft = 0; ft < 8; ft++) {
-        bool first = true; // the first group of f component ft starts a new band block
-        for (int c0 = 0; c0 < M; c0 += 64) {
-            const int i = c0 + lane;
-            const unsigned m = (i < M) ? smask[ft * M + i] : 0u;
-            const unsigned long long bal = __ballot(m != 0);
-            if (m) {
+        const int first = base; // the first group of f component ft starts a new band block
+        for (int c = 0; 64 * c < M; c++) {
+            const int n = s_cnt[ft][c];
+            if (n && c % kScreenWaves == wv) {
+                const int i = 64 * c + lane;
+                const unsigned m = (i < M) ? smask[ft * M + i] : 0u;
+                const unsigned long long bal = __ballot(m != 0);
                 const int rank = __popcll(bal & below);
-                dst[base + rank] = group_code(sb40[i], ft, m, first && rank == 0);
+                if (m) dst[base + rank] = group_code(sb40[i], ft, m, base == first && rank == 0);
             }
-            if (bal) first = false;
-            base += __popcll(bal);
+            base += n;
         }
     }
-    if (lane == 0) gcount[p] = base;
+    if (threadIdx.x == 0) gcount[p] = base;
 }
 
 // ---------------------------------------------------------------------------
@@ -1263,7 +1276,7 @@ template <int N1> struct BandL {
                              w.pdl.as<int4>(), w.pfo.as<long long>(), w.partial.as<double>(), precision, N3};
         {
             ProfileScope prof_(MWG_KERNEL_GROUPS);
-            hipLaunchKernelGGL(k_group_screen, dim3(npairs), dim3(64 * kScreenWaves), 0, 0, dev.segs, dev.node_seg, lvl->l, lvl->node_thr, *pr,
+            hipLaunchKernelGGL(mg.pair ? k_group_screen<true> : k_group_screen<false>, dim3(npairs), dim3(64 * kScreenWaves), 0, 0, dev.segs, dev.node_seg, lvl->l, lvl->node_thr, *pr,
                                w.codes.as<unsigned>(), stride, gstart, w.pdl.as<int4>(), w.pfo.as<long long>(), w.papp.as<int>(), mg);
             MWG_LAUNCHED();
             if (npairs <= kPlanPairs && L <= kPlanNodes) {
