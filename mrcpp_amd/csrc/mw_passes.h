@@ -123,11 +123,12 @@ template <int N1> struct MwMap {
 };
 struct MwNoMap {};
 
-enum MwMapped { MW_NO_MAP, MW_MAP_BEFORE, MW_MAP_AFTER };
+enum MwMapped { MW_NO_MAP, MW_MAP_BEFORE, MW_MAP_AFTER, MW_APART };
 
 // One pass in direction DIM.  in(block, r, i): the input values; out(q, J,
-// block, j, r, v): the outputs, q and J counting a lane's own.  Every thread of
-// the workgroup calls; barriers are the caller's.
+// block, j, r, v): the outputs, q and J counting a lane's own; with MW_APART
+// out(q, J, block, j, r, v0, v1), the sums over either child not yet added.
+// Every thread of the workgroup calls; barriers are the caller's.
 template <int N1, int DIM, MwMapped MAP = MW_NO_MAP, class Map = MwNoMap, class In, class Out>
 __device__ __forceinline__ void mw_pass(const MwMatrix<N1> &M, In in, Out out, const Map &map = Map()) {
     using P = MwShape<N1>;
@@ -152,7 +153,7 @@ __device__ __forceinline__ void mw_pass(const MwMatrix<N1> &M, In in, Out out, c
 #pragma unroll
             for (int J = 0; J < T; J++) a[J] = t[J];
         }
-        double d[T];
+        double d[T], e[MAP == MW_APART ? T : 1];
 #pragma unroll
         for (int J = 0; J < T; J++) {
             double d0 = 0.0, d1 = 0.0;
@@ -162,15 +163,24 @@ __device__ __forceinline__ void mw_pass(const MwMatrix<N1> &M, In in, Out out, c
                 if (4 * K < N1) d0 = __builtin_amdgcn_mfma_f64_4x4x4f64(M.m[J][K], lo, d0, 0, 0, 0);
                 if (4 * K + 3 >= N1) d1 = __builtin_amdgcn_mfma_f64_4x4x4f64(M.m[J][K], hi, d1, 0, 0, 0);
             }
-            d[J] = d0 + d1;
+            if constexpr (MAP == MW_APART) {
+                d[J] = d0;
+                e[J] = d1;
+            } else {
+                d[J] = d0 + d1;
+            }
             if constexpr (N1 == 10) __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
         for (int J = 0; J < T; J++) {
             const int o = 4 * J + kk, b = o >= N1;
-            double v = d[J];
-            if constexpr (MAP == MW_MAP_AFTER) v = map.tile(J, d, lane);
-            out(q, J, blk | b << DIM, o - b * N1, r, v);
+            if constexpr (MAP == MW_APART) {
+                out(q, J, blk | b << DIM, o - b * N1, r, d[J], e[J]);
+            } else {
+                double v = d[J];
+                if constexpr (MAP == MW_MAP_AFTER) v = map.tile(J, d, lane);
+                out(q, J, blk | b << DIM, o - b * N1, r, v);
+            }
         }
     }
 }

@@ -107,9 +107,10 @@ __global__ __launch_bounds__(MwShape<N1>::THREADS, MwShape<N1>::OCC) void k_reco
     __syncthreads();
     mw_pass_lds<N1, 1>(b, a, M);
     __syncthreads();
-    mw_pass<N1, 2>(
+    // the two contributions added one after the other
+    mw_pass<N1, 2, MW_APART>(
         M, [&](int t, int r, int i) { return b[P::at(t, r, i)]; },
-        [&](int q, int J, int t, int j, int r, double v) { dst[t * stride + j * P::N2 + r] = old[q][J] + v; });
+        [&](int q, int J, int t, int j, int r, double v0, double v1) { dst[t * stride + j * P::N2 + r] = old[q][J] + v0 + v1; });
 }
 
 template <int N1>
