@@ -17,8 +17,8 @@
 //     other matrix-core cases) or k_band_units (vector ALUs): persistent
 //     workgroups take units in turn or from an atomic counter; a unit
 //     accumulates its groups' 3-sweep tensor products in registers and writes
-//     one 8-block result, into partial slots or, as a node's only unit (with
-//     the latter two kernels also as its first), the output coefficients.
+//     one 8-block result, the node's first unit straight into the output
+//     coefficients, later units into partial slots.
 //  4. k_reduce_waves / k_reduce_units: per output node and chunk of
 //     coefficients, the partial slots are added in unit order; k_level_norms computes the component
 //     norms (MWNode::calcNorms, src/trees/MWNode.cpp:609-655).
@@ -263,14 +263,13 @@ __device__ inline int units_group_size(int gmin, int total, int slots, int T) {
 }
 
 // Units per output node, packed with a flag so one scan yields both the first
-// unit and the first partial slot of every node.  With all_slots (the wave
-// kernels) a node of several units has a slot for each, else for each but the
-// first, which writes the node itself; the flag marks the units without one.
+// unit and the first partial slot of every node: the first unit writes the node
+// itself, each further one has a slot.
 // The node has np pairs from gf on, with T groups and app applied tuples, total
 // groups in the level.  Every thread of a wave calls, with node g live or not; the
 // node's counters and margins are added up on the way.
 __device__ __forceinline__ long long node_units(int g, bool live, int gf, int np, int T, unsigned long long app, int total, int gmin, int slots,
-                                                bool all_slots, const mwg_segment *segs, const int *node_seg, const double *pmg, double *g_margin) {
+                                                const mwg_segment *segs, const int *node_seg, const double *pmg, double *g_margin) {
     // applied tuples and candidate pairs of the node's pairs, added to its
     // segment's counters: one atomic per wave when the wave's nodes share a
     // segment (lane 0 holds the wave's first node)
@@ -303,10 +302,10 @@ __device__ __forceinline__ long long node_units(int g, bool live, int gf, int np
     }
     const int G = units_group_size(gmin, total, slots, T);
     const int nu = (T + G - 1) / G;
-    return (long long)nu + ((long long)(all_slots ? nu == 1 : nu > 0) << 32);
+    return (long long)nu + ((long long)(nu > 0) << 32);
 }
 
-__global__ __launch_bounds__(256) void k_unit_count(int L, mwg_pairs pr, int npairs, const int *gstart, int gmin, int slots, bool all_slots, long long *packed, int *counter,
+__global__ __launch_bounds__(256) void k_unit_count(int L, mwg_pairs pr, int npairs, const int *gstart, int gmin, int slots, long long *packed, int *counter,
                                                     const mwg_segment *segs, const int *node_seg, const int *papp, const double *pmg, double *g_margin) {
     const int g = blockIdx.x * 256 + threadIdx.x;
     if (g == 0) *counter = 0;
@@ -314,7 +313,7 @@ __global__ __launch_bounds__(256) void k_unit_count(int L, mwg_pairs pr, int npa
     const int gf = live ? pr.g_first[g] : 0, np = live ? pr.g_npairs[g] : 0;
     unsigned long long app = 0;
     for (int q = gf; q < gf + np; q++) app += (unsigned)papp[q];
-    const long long v = node_units(g, live, gf, np, live ? gstart[gf + np] - gstart[gf] : 0, app, gstart[npairs], gmin, slots, all_slots, segs, node_seg,
+    const long long v = node_units(g, live, gf, np, live ? gstart[gf + np] - gstart[gf] : 0, app, gstart[npairs], gmin, slots, segs, node_seg,
                                    pmg, g_margin);
     if (live) packed[g] = v;
 }
@@ -327,7 +326,7 @@ __global__ __launch_bounds__(256) void k_unit_count(int L, mwg_pairs pr, int npa
 // The bounds are what one workgroup's LDS and threads hold; at them the work is
 // spread over more workgroups anyway.
 constexpr int kPlanPairs = 16384, kPlanNodes = 1024;
-__global__ __launch_bounds__(kPlanNodes) void k_unit_plan(int L, mwg_pairs pr, int npairs, int *gstart, int gmin, int slots, bool all_slots, long long *packed, int *counter,
+__global__ __launch_bounds__(kPlanNodes) void k_unit_plan(int L, mwg_pairs pr, int npairs, int *gstart, int gmin, int slots, long long *packed, int *counter,
                                                           const mwg_segment *segs, const int *node_seg, const int *papp, const double *pmg,
                                                           double *g_margin) {
     // groups of a pair, applied tuples in the upper half; then before a pair
@@ -356,7 +355,7 @@ __global__ __launch_bounds__(kPlanNodes) void k_unit_plan(int L, mwg_pairs pr, i
     __syncthreads();
     for (int q = tid; q <= npairs; q += kPlanNodes) gstart[q] = (int)(unsigned)gs[at(q)];
     const unsigned long long mine = gs[at(gf + np)] - gs[at(gf)];
-    const long long v = node_units(tid, live, gf, np, (int)(unsigned)mine, mine >> 32, (int)(unsigned)total, gmin, slots, all_slots, segs, node_seg, pmg,
+    const long long v = node_units(tid, live, gf, np, (int)(unsigned)mine, mine >> 32, (int)(unsigned)total, gmin, slots, segs, node_seg, pmg,
                                    g_margin);
     long long units;
     const long long all = block_exclusive_scan<long long, kPlanNodes>(v, tl, units);
@@ -367,52 +366,32 @@ __global__ __launch_bounds__(kPlanNodes) void k_unit_plan(int L, mwg_pairs pr, i
 __device__ inline int unit_first(long long v) { return (int)(v & 0xffffffffll); }
 __device__ inline int flagged_before(long long v) { return (int)(v >> 32); }
 
-// What a wave kernel reads of a unit and of a group, written here so that it
-// needs no chain of lookups.  Unit (three int4): operand table, band
-// coefficient pool and result address (64 bits each), first group, number of
-// groups, whether the result is the output node itself.  Group (one int4, level
-// order): x block | gt mask << 24, y block | f bits 32-42 << 21, z block | f
-// bits 43-53 << 21, f bits 0-31; a block is 2 (b40 + dl) + f bit of its
-// direction (21 bits), f the offset of the group's band block.
+// What a wave kernel reads of a unit, written here so that it needs no chain of
+// lookups (three int4): operand table, band coefficient pool and result address
+// (64 bits each), first group, number of groups, whether the result is written in
+// the output node's order.
 struct WaveRecords {
-    int4 *unit, *group; // null: not a wave kernel
+    int4 *unit; // null: not a wave kernel
     const mwg_segment *segs;
     const int *node_seg;
     const long long *g_off;
-    const int4 *pdl;
-    const long long *pfo;
     double *partial;
     int prec, n3;
+    bool in_place; // the first of several units writes the node in the slots' order
 };
 constexpr int kUnitInts = 12;
 
 // One wave per pair: the descriptors of the units that start inside the pair
 // ({pair, first group in the pair, groups, partial slot or -1}, or a wave
-// kernel's) and, for the matrix-core kernels, the pair's groups in level order
-// (gstart numbering; grec: code and pair index, or a wave kernel's records).
+// kernel's) and, when grec is given, the pair's group codes in level order
+// (gstart numbering) with the pair index.
 __global__ __launch_bounds__(64) void k_unit_write(int npairs, mwg_pairs pr, const int *gstart, const long long *uscan, int gmin, int slots, int4 *units,
                                                    const unsigned *codes, int stride, int2 *grec, WaveRecords wr) {
     const int p = blockIdx.x;
     const int base = gstart[p], cnt = gstart[p + 1] - base;
     if (cnt == 0) return;
-    if (wr.group) {
-        const int4 d = wr.pdl[p];
-        const long long fo = wr.pfo[p];
-        for (int k = threadIdx.x; k < cnt; k += 64) {
-            const unsigned code = codes[(size_t)p * stride + k];
-            const int ft = code_ft(code), b = code_block(code);
-            const long long f = fo + (long long)ft * wr.n3;
-            const unsigned fh = (unsigned)(f >> 32);
-            int4 r;
-            r.x = (int)((unsigned)((b + d.x) * 2 + (ft & 1)) | (code_mask(code) << 24));
-            r.y = (int)((unsigned)((b + d.y) * 2 + ((ft >> 1) & 1)) | (fh << 21));
-            r.z = (int)((unsigned)((b + d.z) * 2 + ((ft >> 2) & 1)) | ((fh >> 11) << 21));
-            r.w = (int)(unsigned)f;
-            wr.group[base + k] = r;
-        }
-    } else if (grec) {
+    if (grec)
         for (int k = threadIdx.x; k < cnt; k += 64) grec[base + k] = make_int2((int)codes[(size_t)p * stride + k], p);
-    }
     if (threadIdx.x != 0) return;
     const int g = pr.pair_g[p];
     const int gf = pr.g_first[g], np = pr.g_npairs[g];
@@ -432,12 +411,11 @@ __global__ __launch_bounds__(64) void k_unit_write(int npairs, mwg_pairs pr, con
     auto lo = [](const void *q) { return (int)(unsigned)reinterpret_cast<unsigned long long>(q); };
     auto hi = [](const void *q) { return (int)(unsigned)(reinterpret_cast<unsigned long long>(q) >> 32); };
     for (int j = (a + G - 1) / G; j * G < e; j++) {
-        const bool direct = T <= G;
-        const double *out = direct ? node : wr.partial + (size_t)(Sg + j) * 8 * wr.n3;
+        const double *out = j == 0 ? node : wr.partial + (size_t)(Sg + j - 1) * 8 * wr.n3;
         int4 *u = wr.unit + (kUnitInts / 4) * (size_t)(Ug + j);
         u[0] = make_int4(lo(S.op.frag[wr.prec]), hi(S.op.frag[wr.prec]), lo(S.f.coef), hi(S.f.coef));
         u[1] = make_int4(lo(out), hi(out), B + j * G, min(G, T - j * G));
-        u[2] = make_int4(direct ? 1 : 0, 0, 0, 0);
+        u[2] = make_int4(T <= G || (j == 0 && !wr.in_place) ? 1 : 0, 0, 0, 0);
     }
 }
 
@@ -1456,7 +1434,7 @@ template <int N1, int PREC>
 void launch_mfma(const mwg_level *lvl, const LevelDevice &dev, const mwg_pairs *pr, BandWork &w, bool waves) {
     if constexpr (PREC == MWG_PREC_FP64 || (PREC == MWG_PREC_FP32 && N1 == 8)) {
         if (waves) {
-            const WaveArgs a{w.grec.as<int4>(), w.units.as<int>(), w.uscan.as<long long>(), lvl->count};
+            const WaveArgs a{w.grec.as<int2>(), w.pdl.as<int4>(), w.pfo.as<long long>(), w.units.as<int>(), w.uscan.as<long long>(), lvl->count};
             hipLaunchKernelGGL((wave_kernel_of<N1, PREC>()), dim3(wave_grid<N1, PREC>()), dim3(wave_threads<N1>()), 0, 0, a);
             return;
         }
@@ -1500,12 +1478,10 @@ template <int N1> struct BandL {
         if (w.uscan.ensure(sizeof(long long) * ((size_t)L + 1)) != MWG_OK) return MWG_ERR_NOMEM;
         const bool waves = wave_kernel(N1, precision, npairs);
         if (w.units.ensure((waves ? sizeof(int) * kUnitInts : sizeof(int4)) * ((size_t)slots + L)) != MWG_OK) return MWG_ERR_NOMEM;
-        // with all_slots a node of several units (more than one per slot's
-        // share of groups, so at most `slots` of them) takes one more
-        if (w.partial.ensure(slot_bytes * ((size_t)slots + (waves ? std::min(slots, L) : 0))) != MWG_OK) return MWG_ERR_NOMEM;
+        if (w.partial.ensure(slot_bytes * (size_t)slots) != MWG_OK) return MWG_ERR_NOMEM;
         if (w.counter.ensure(sizeof(int)) != MWG_OK) return MWG_ERR_NOMEM;
         const bool mfma = precision != kPrecValuBand;
-        if (mfma && w.grec.ensure((waves ? sizeof(int4) : sizeof(int2)) * (size_t)npairs * stride) != MWG_OK) return MWG_ERR_NOMEM;
+        if (mfma && w.grec.ensure(sizeof(int2) * (size_t)npairs * stride) != MWG_OK) return MWG_ERR_NOMEM;
         if (w.pdl.ensure(sizeof(int4) * (size_t)npairs) != MWG_OK) return MWG_ERR_NOMEM;
         if (w.pfo.ensure(sizeof(long long) * (size_t)npairs) != MWG_OK) return MWG_ERR_NOMEM;
         if (w.papp.ensure(sizeof(int) * (size_t)npairs) != MWG_OK) return MWG_ERR_NOMEM;
@@ -1517,21 +1493,21 @@ template <int N1> struct BandL {
         }
         int *gstart = w.gstart.as<int>();
         long long *uscan = w.uscan.as<long long>();
-        const WaveRecords wr{waves ? w.units.as<int4>() : nullptr, waves ? w.grec.as<int4>() : nullptr, dev.segs, dev.node_seg, lvl->g_off,
-                             w.pdl.as<int4>(), w.pfo.as<long long>(), w.partial.as<double>(), precision, N3};
+        const WaveRecords wr{waves ? w.units.as<int4>() : nullptr, dev.segs, dev.node_seg, lvl->g_off, w.partial.as<double>(), precision, N3,
+                             WaveMap<N1, MWG_PREC_FP64>::IN_PLACE};
         {
             ProfileScope prof_(MWG_KERNEL_GROUPS);
             hipLaunchKernelGGL(mg.pair ? k_group_screen<true> : k_group_screen<false>, dim3(npairs), dim3(64 * kScreenWaves), 0, 0, dev.segs, dev.node_seg, lvl->l, lvl->node_thr, *pr,
                                w.codes.as<unsigned>(), stride, gstart, w.pdl.as<int4>(), w.pfo.as<long long>(), w.papp.as<int>(), mg);
             MWG_LAUNCHED();
             if (npairs <= kPlanPairs && L <= kPlanNodes) {
-                hipLaunchKernelGGL(k_unit_plan, dim3(1), dim3(kPlanNodes), 0, 0, L, *pr, npairs, gstart, g_unit_groups, slots, waves, uscan,
+                hipLaunchKernelGGL(k_unit_plan, dim3(1), dim3(kPlanNodes), 0, 0, L, *pr, npairs, gstart, g_unit_groups, slots, uscan,
                                    w.counter.as<int>(), dev.segs, dev.node_seg, w.papp.as<int>(), mg.pair, lvl->g_margin);
                 MWG_LAUNCHED();
             } else {
                 mwg_status s = scan_exclusive(gstart, gstart, npairs);
                 if (s != MWG_OK) return s;
-                hipLaunchKernelGGL(k_unit_count, dim3((L + 255) / 256), dim3(256), 0, 0, L, *pr, npairs, gstart, g_unit_groups, slots, waves, uscan,
+                hipLaunchKernelGGL(k_unit_count, dim3((L + 255) / 256), dim3(256), 0, 0, L, *pr, npairs, gstart, g_unit_groups, slots, uscan,
                                    w.counter.as<int>(), dev.segs, dev.node_seg, w.papp.as<int>(), mg.pair, lvl->g_margin);
                 MWG_LAUNCHED();
                 s = scan_exclusive(uscan, uscan, L);
@@ -1560,8 +1536,9 @@ template <int N1> struct BandL {
             const dim3 rgrid(L, (8 * N3 + 255) / 256);
             if constexpr (N1 == 8) {
                 if (waves) {
-                    hipLaunchKernelGGL(precision == MWG_PREC_FP64 ? k_reduce_waves8<MWG_PREC_FP64> : k_reduce_waves8<MWG_PREC_FP32>, dim3(L, 4), dim3(1024),
-                                       0, 0, dev.segs, dev.node_seg, lvl->g_off, uscan, w.partial.as<double>());
+                    const int rows = precision == MWG_PREC_FP64 ? WaveMap<8, MWG_PREC_FP64>::SET : WaveMap<8, MWG_PREC_FP32>::SET;
+                    hipLaunchKernelGGL(precision == MWG_PREC_FP64 ? k_reduce_waves8<MWG_PREC_FP64> : k_reduce_waves8<MWG_PREC_FP32>, dim3(L, 64 / rows),
+                                       dim3(64 * rows), 0, 0, dev.segs, dev.node_seg, lvl->g_off, uscan, w.partial.as<double>());
                     MWG_LAUNCHED();
                     hipLaunchKernelGGL(k_level_norms<N1>, dim3(L), dim3(kThreads), 0, 0, dev.segs, dev.node_seg, lvl->g_off, lvl->g_norms);
                     MWG_LAUNCHED();
@@ -1578,7 +1555,7 @@ template <int N1> struct BandL {
             }
             if constexpr (N1 == 6 || N1 == 10) {
                 if (waves)
-                    hipLaunchKernelGGL(k_reduce_waves<N1>, rgrid, dim3(256), 0, 0, dev.segs, dev.node_seg, lvl->g_off, uscan, w.partial.as<double>());
+                    hipLaunchKernelGGL(k_reduce_waves<N1>, dim3(L, WaveShape<N1>::VALS), dim3(64 * WaveShape<N1>::ITEMS), 0, 0, dev.segs, dev.node_seg, lvl->g_off, uscan, w.partial.as<double>());
             }
             if (!waves)
                 hipLaunchKernelGGL(k_reduce_units<N1>, rgrid, dim3(256), 0, 0, dev.segs, dev.node_seg, lvl->g_off, uscan, w.partial.as<double>());

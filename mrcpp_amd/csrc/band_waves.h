@@ -31,10 +31,11 @@
 // multiply-add per contracted index, in index order, whichever instruction
 // shape forms them), so order 7 gives the same bits with either.
 //
-// Results: a node of one unit is written to its output block; a node of
-// several units has a slot per unit, in the order of WaveMap, which each wave
-// writes in whole 512-byte rows (the reductions add the slots in unit order
-// and put the sums in place).
+// Results: a node's first unit is written to the node itself, each further unit
+// to a slot in the order of WaveMap, which each wave writes in whole 512-byte
+// rows; the reductions add the slots to the node in unit order.  The first of
+// several units writes the node in the slots' order too where a workgroup of the
+// reduction can put it right in place (orders 3 and 7).
 #pragma once
 
 namespace mwgdev {
@@ -55,11 +56,22 @@ template <int N1> struct WaveShape {
     static constexpr int VALS = 8 * N3 / (64 * ITEMS);  // result values per lane of an item
 };
 
-// Output element (gt block, j0, j1, j2) of value e (register index, lane) of
-// item `it`: the layout of the partial slots, slot[(it * VALS + v) * 64 + lane].
+// Value v (register index) of item `it`: row(it, v), its 64 lanes' place in a
+// partial slot, slot[64 row + lane]; out(it, v, lane), a lane's output element
+// (gt block, j0, j1, j2).  At order 7 the four (FP64) or eight (FP32) rows that
+// hold every j0 and j1 of their outputs lie where those outputs lie in a node, at
+// orders 5 and 9 the rows of every j0 follow each other.
 template <int N1, int PREC> struct WaveMap {
     using S = WaveShape<N1>;
     static constexpr int TC = N1 / 2; // tiles of four columns or rows of one 2 N1 side
+    static constexpr bool IN_PLACE = N1 == 4 || N1 == 8;
+    static constexpr int SET = N1 != 8 ? S::ITEMS : PREC == MWG_PREC_FP64 ? 4 : 8; // rows of a workgroup of the reduction
+    __device__ static inline int row(int it, int v) {
+        if constexpr (N1 != 8) return v * S::ITEMS + it;
+        const int gx = it >> 1, half = it & 1, t = v >> 2, r = v & 3;
+        if constexpr (PREC == MWG_PREC_FP64) return (gx + 2 * (t & 1) + 4 * (r >> 1)) * 8 + 4 * (r & 1) + 2 * half + (t >> 1);
+        return (gx + 2 * t) * 8 + 4 * half + r;
+    }
     __device__ static inline int out(int it, int v, int lane) {
         int gx, gy, gz, j0, j1, j2;
         if constexpr (N1 == 8) {
@@ -93,8 +105,10 @@ template <int N1, int PREC> struct WaveMap {
 };
 
 struct WaveArgs {
-    const int4 *group; // WaveRecords
-    const int *unit;
+    const int2 *group; // group codes and pair indices, level order
+    const int4 *pdl;   // of a pair: translation differences, offset of the band node
+    const long long *pfo;
+    const int *unit; // WaveRecords
     const long long *uscan;
     int L;
 };
@@ -107,21 +121,23 @@ struct WaveGroup {
 };
 
 // The groups of a work unit that touch the wave's columns (bits `want` of
-// their gt masks), in order.  64 records at a time in registers, lane j
-// holding group c0 + j.  Units are dealt out in turn: one shared counter served
-// a small level's waves more slowly than they worked (86 us a launch at order 3
-// against 20).
-struct WaveUnit {
-    const int4 *group;
+// their gt masks), in order.  64 at a time in registers, lane j holding group
+// c0 + j: x block | gt mask << 24, y block | f bits 32-42 << 21, z block | f bits
+// 43-53 << 21, f bits 0-31; a block is 2 (b40 + dl) + f bit of its direction (21
+// bits), f the offset of the group's band block.  Units are dealt out in turn: one
+// shared counter served a small level's waves more slowly than they worked (86 us
+// a launch at order 3 against 20).
+template <int N1> struct WaveUnit {
+    const WaveArgs &a;
     unsigned long long frag, coef; // operand table, coefficient pool
-    global<double> *out;           // result: the unit's slot or (direct) the output node
+    global<double> *out;           // result: the unit's slot or the output node
     int gi0, ng, c0;
     unsigned want;
     bool direct;
     int4 rec;
     unsigned long long todo;
 
-    __device__ WaveUnit(const WaveArgs &a, int u, unsigned want_, int lane) : group(a.group), c0(0), want(want_ << 24) {
+    __device__ WaveUnit(const WaveArgs &a_, int u, unsigned want_, int lane) : a(a_), c0(0), want(want_ << 24) {
         const auto d = ro(a.unit) + kUnitInts * (size_t)u;
         auto ptr = [](int lo, int hi) { return ((unsigned long long)(unsigned)hi << 32) | (unsigned)lo; };
         frag = ptr(d[0], d[1]);
@@ -134,7 +150,18 @@ struct WaveUnit {
     }
     __device__ void load(int lane) {
         rec = int4{0, 0, 0, 0};
-        if (c0 + lane < ng) rec = group[gi0 + c0 + lane];
+        if (c0 + lane < ng) {
+            const int2 g = a.group[gi0 + c0 + lane];
+            const int4 d = a.pdl[g.y];
+            const unsigned code = (unsigned)g.x;
+            const int ft = code_ft(code), b = code_block(code);
+            const long long f = a.pfo[g.y] + (long long)ft * (N1 * N1 * N1);
+            const unsigned fh = (unsigned)(f >> 32);
+            rec.x = (int)((unsigned)((b + d.x) * 2 + (ft & 1)) | (code_mask(code) << 24));
+            rec.y = (int)((unsigned)((b + d.y) * 2 + ((ft >> 1) & 1)) | (fh << 21));
+            rec.z = (int)((unsigned)((b + d.z) * 2 + ((ft >> 2) & 1)) | ((fh >> 11) << 21));
+            rec.w = (int)(unsigned)f;
+        }
         todo = __ballot(((unsigned)rec.x & want) != 0u);
     }
     __device__ bool next(int lane, WaveGroup &q) {
@@ -157,7 +184,7 @@ struct WaveUnit {
     }
 };
 
-// An item's result values into the unit's slot or the output node.
+// An item's result values into the unit's slot or the output node, in the node's order (direct) or the slots'.
 template <int N1, int PREC, typename V> __device__ inline void wave_store(global<double> *out, bool direct, int it, int lane, V &&value) {
     constexpr int VALS = WaveShape<N1>::VALS;
     asm volatile("" : "+v"(lane)); // the addresses are formed here, not kept in registers over the groups
@@ -166,7 +193,7 @@ template <int N1, int PREC, typename V> __device__ inline void wave_store(global
         for (int v = 0; v < VALS; v++) out[WaveMap<N1, PREC>::out(it, v, lane)] = value(v);
     } else {
 #pragma unroll
-        for (int v = 0; v < VALS; v++) out[(it * VALS + v) * 64 + lane] = value(v);
+        for (int v = 0; v < VALS; v++) out[WaveMap<N1, PREC>::row(it, v) * 64 + lane] = value(v);
     }
 }
 
@@ -212,7 +239,7 @@ __global__ __launch_bounds__(256, 4) void k_band_waves8(WaveArgs a) {
         double x[2], y[2][2], z[2];
     };
     for (int unit = blockIdx.x; unit < total; unit += gridDim.x) {
-        WaveUnit w(a, unit, 0x55u << gx, lane);
+        WaveUnit<8> w(a, unit, 0x55u << gx, lane);
         dvec4 acc[2][2];
 #pragma unroll
         for (int t = 0; t < 4; t++) acc[t >> 1][t & 1] = dvec4{0.0, 0.0, 0.0, 0.0};
@@ -318,7 +345,7 @@ __global__ __launch_bounds__(256, 4) void k_band_waves8f(WaveArgs a) {
         float x[8], y[2], z[2];
     };
     for (int unit = blockIdx.x; unit < total; unit += gridDim.x) {
-        WaveUnit w(a, unit, 0x55u << gx, lane);
+        WaveUnit<8> w(a, unit, 0x55u << gx, lane);
         dvec4 acc[4];
 #pragma unroll
         for (int t = 0; t < 4; t++) acc[t] = dvec4{0.0, 0.0, 0.0, 0.0};
@@ -449,7 +476,7 @@ template <int N1> __global__ __launch_bounds__(64, WaveLds<N1>::WAVES) void k_ba
     // operand table offset of column n, contracted index 4 ks + lq
     auto at = [&](int n, int ks) { return (ks * NT + (n >> 4)) * 64 + (n & 15) + 16 * lq; };
     for (int unit = turn.unit; unit < total; unit += turn.step) {
-        WaveUnit w(a, unit, 0xffu, lane);
+        WaveUnit<N1> w(a, unit, 0xffu, lane);
         const auto frag = (const global<double> *)w.frag;
         double acc[PW][TC][TC];
 #pragma unroll
@@ -621,70 +648,61 @@ template <int N1> __global__ __launch_bounds__(64, WaveLds<N1>::WAVES) void k_ba
     }
 }
 
-// Slots of the nodes of more than one unit added in unit order, eight slots'
-// loads in flight: v0 + v1 + ... of one value, src[j stride] that of slot j.
-__device__ __forceinline__ double slot_sum(const double *src, int nu, size_t stride) {
-    double acc = src[0];
-    int j = 1;
-    for (; j + 8 <= nu; j += 8) {
+// Partial slots of a node added to its first unit's value in unit order, eight
+// slots' loads in flight: src[j stride] is slot j's value.
+__device__ __forceinline__ double slot_sum(double acc, const double *src, int slots, size_t stride) {
+    int j = 0;
+    for (; j + 8 <= slots; j += 8) {
         double t[8];
 #pragma unroll
         for (int q = 0; q < 8; q++) t[q] = src[(size_t)(j + q) * stride];
 #pragma unroll
         for (int q = 0; q < 8; q++) acc += t[q];
     }
-    for (; j < nu; j++) acc += src[(size_t)j * stride];
+    for (; j < slots; j++) acc += src[(size_t)j * stride];
     return acc;
 }
 
-// A thread per value of the slots' layout (orders 5 and 9).
+// Orders 5 and 9: a workgroup takes the same value of every item.
 template <int N1>
-__global__ __launch_bounds__(256) void k_reduce_waves(const mwg_segment *segs, const int *node_seg, const long long *g_off, const long long *uscan,
-                                                      const double *partial) {
-    using W = WaveShape<N1>;
+__global__ __launch_bounds__(64 * WaveShape<N1>::ITEMS) void k_reduce_waves(const mwg_segment *segs, const int *node_seg, const long long *g_off,
+                                                                            const long long *uscan, const double *partial) {
+    constexpr int N = 8 * WaveShape<N1>::N3;
     const int g = blockIdx.x;
-    const int e = blockIdx.y * 256 + threadIdx.x;
     const long long v = uscan[g];
     const int Ug = unit_first(v);
     const int nu = unit_first(uscan[g + 1]) - Ug;
-    if (nu == 1 || e >= 8 * W::N3) return; // a single unit wrote the node already
-    double *dst = ro(segs)[ro(node_seg)[g]].g_coef + g_off[g];
-    const int o = WaveMap<N1, MWG_PREC_FP64>::out((e >> 6) / W::VALS, (e >> 6) % W::VALS, e & 63);
-    dst[o] = nu == 0 ? 0.0 : slot_sum(partial + (size_t)(Ug - flagged_before(v)) * 8 * W::N3 + e, nu, 8 * W::N3);
+    if (nu == 1) return; // a single unit wrote the node already
+    double *dst = ro(segs)[ro(node_seg)[g]].g_coef + g_off[g] + WaveMap<N1, MWG_PREC_FP64>::out(threadIdx.x >> 6, blockIdx.y, threadIdx.x & 63);
+    *dst = nu == 0 ? 0.0 : slot_sum(*dst, partial + (size_t)(Ug - flagged_before(v)) * N + blockIdx.y * blockDim.x + threadIdx.x, nu - 1, N);
 }
 
-// Order 7: a workgroup takes the 16 rows of the slots that hold every j0 and j1
-// of its outputs, (gx, gy) at FP64, gx and the j2 of two residues mod 4 at FP32,
-// and hands them through LDS into whole 512-byte runs of the node (written one
-// by one from the slots' order, a level's nodes are reached in pieces of 16 bytes:
-// FP32, 32 Gaussians, 1.92 -> 1.61 ms).
+// Order 7: a workgroup takes the rows that hold every j0 and j1 of their outputs,
+// those of one (gx, gy, r) at FP64, of one (gx, r) at FP32, adds them up and puts
+// them in place through LDS (written one by one from the slots' order a level's
+// nodes are reached in pieces of 16 bytes).  256 or 512 threads a workgroup: an
+// application to 32 Gaussians at FP64 takes 1.59 ms of it (1.75 with 1024 and a slot
+// for the first unit, 1.56 for k_reduce_units after the kernel by rows).
 template <int PREC>
-__global__ __launch_bounds__(1024) void k_reduce_waves8(const mwg_segment *segs, const int *node_seg, const long long *g_off, const long long *uscan,
-                                                        const double *partial) {
-    using W = WaveShape<8>;
+__global__ __launch_bounds__((64 * WaveMap<8, PREC>::SET)) void k_reduce_waves8(const mwg_segment *segs, const int *node_seg, const long long *g_off,
+                                                                                const long long *uscan, const double *partial) {
+    using M = WaveMap<8, PREC>;
     constexpr bool F64 = PREC == MWG_PREC_FP64;
-    __shared__ double c[1024];
+    __shared__ double c[64 * M::SET];
     const int g = blockIdx.x, y = blockIdx.y, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const long long v = uscan[g];
     const int Ug = unit_first(v);
     const int nu = unit_first(uscan[g + 1]) - Ug;
     if (nu == 1) return; // a single unit wrote the node already
-    // runs of 64 outputs: FP64 (gz, j2), FP32 (gy, gz, j2 / 4, j2 % 2)
-    const auto run = [&](int o) { return F64 ? (o >> 11 << 3) | (o >> 6 & 7) : (o >> 10 << 2) | (o >> 8 & 1) << 1 | (o >> 6 & 1); };
-    double x = 0.0;
-    const int gx = y >> 1;
-    // item 2 gx + w / 8; value t * 4 + r of it
-    const int it = 2 * gx + (w >> 3);
-    const int val = F64 ? 4 * (2 * (w >> 2 & 1) + (y & 1)) + (w & 3) : 4 * (w >> 1 & 3) + 2 * (y & 1) + (w & 1);
-    const int o = WaveMap<8, PREC>::out(it, val, lane);
-    if (nu > 1) x = slot_sum(partial + (size_t)(Ug - flagged_before(v)) * 4096 + (it * W::VALS + val) * 64 + lane, nu, 4096);
-    c[run(o) * 64 + (o & 63)] = x;
-    __syncthreads();
-    // run w of the workgroup, as a node offset
-    const int base = F64 ? ((gx + 2 * (y & 1) + 4 * (w >> 3)) << 9) + ((w & 7) << 6)
-                         : ((gx + 2 * (w >> 2 & 1) + 4 * (w >> 3)) << 9) + ((4 * (w >> 1 & 1) + 2 * (y & 1) + (w & 1)) << 6);
+    const int r = y & 3, gx = F64 ? y >> 3 : y >> 2;
+    const int it = 2 * gx + (F64 ? w >> 1 : w >> 2), val = F64 ? 4 * (2 * (w & 1) + (y >> 2 & 1)) + r : 4 * (w & 3) + r;
+    const int e = M::row(it, val) * 64 + lane, o = M::out(it, val, lane);
     double *dst = ro(segs)[ro(node_seg)[g]].g_coef + g_off[g];
-    dst[base + lane] = c[threadIdx.x];
+    // the row of the workgroup that lies where output o does
+    const int at = F64 ? o >> 6 & 3 : (o >> 10 & 3) | (o >> 8 & 1) << 2;
+    c[64 * at + (o & 63)] = nu == 0 ? 0.0 : slot_sum(dst[e], partial + (size_t)(Ug - flagged_before(v)) * 4096 + e, nu - 1, 4096);
+    __syncthreads();
+    dst[e] = c[threadIdx.x];
 }
 
 // The same at order 3 with the component norms (block_norms' order) in one
@@ -706,12 +724,11 @@ __global__ __launch_bounds__(512) void k_reduce_norms(const mwg_segment *segs, c
     if (nu == 1) {
         c[e] = dst[e];
     } else {
-        const int o = WaveMap<4, MWG_PREC_FP64>::out((e >> 6) / W::VALS, (e >> 6) % W::VALS, e & 63);
-        const double x = nu == 0 ? 0.0 : slot_sum(partial + (size_t)(Ug - flagged_before(v)) * 512 + e, nu, 512);
-        c[o] = x;
-        dst[o] = x;
+        const int o = WaveMap<4, MWG_PREC_FP64>::out((e >> 6) % W::ITEMS, (e >> 6) / W::ITEMS, e & 63);
+        c[o] = nu == 0 ? 0.0 : slot_sum(dst[e], partial + (size_t)(Ug - flagged_before(v)) * 512 + e, nu - 1, 512);
     }
     __syncthreads();
+    if (nu != 1) dst[e] = c[e];
     block_norms<4>(c, g_norms + (size_t)g * 9, red);
 }
 
