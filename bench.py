@@ -28,9 +28,9 @@ METRIC = "Poisson apply s/tree + GFLOP/s (order 7, \u03b5=1e-6), chosen vs plain
 
 
 def band_kernel(precision, order=7):
-    """Family of the band kernel that runs: the one-wave-per-item kernels for
-    FP64 at every order and FP32 at order 7 (unless the tile layout is selected
-    there), the tile-shared one otherwise."""
+    """Family of the band kernel that a single tree runs: the one-wave-per-item
+    kernels for FP64 at every order and FP32 at order 7 (unless the tile layout is
+    selected there), the tile-shared one otherwise."""
     import mrcpp_amd as mr
     if (precision == "fp64" and order != 7) or (order == 7 and precision in ("fp64", "fp32") and mr.band_layout() != "tiles"):
         return "k_band_waves"
@@ -420,7 +420,8 @@ def batch_bench(args, steps, warmup):
         "speedup_vs_plain": round(p_s / c_s, 3),
         "error_vs_plain_fp64": {"rel_l2_same_trees": (num / den) ** 0.5 if den > 0 else None, "same_node_set_trees": same, "trees": n,
                                 "applied_chosen": int(sum(st["n_applied"] for st in c_sts))},
-        "roofline": {"bound": "mfma", "kernel": band_kernel(args.precision), "achieved": round(c_flop / (band_ms_per_step / 1e3) / 1e12, 4),
+        # a batch's long levels take the kernel by rows
+        "roofline": {"bound": "mfma", "kernel": band_kernel(args.precision).replace("waves", "rows, k_band_waves"), "achieved": round(c_flop / (band_ms_per_step / 1e3) / 1e12, 4),
                      "peak": FP64_PEAK_TFLOPS if args.precision in ("fp64", "fp64_vector") else 157.3, "unit": "TFLOP/s",
                      "launches_per_step": band_launches / (steps + max(warmup, 1))},
         "kernel_ms_per_step": {k: round(v[0], 4) for k, v in every.items()},

@@ -366,9 +366,11 @@ mwg_status mwg_hash_update_multi(const mwg_hash_table *tables, int ntables, cons
 mwg_status mwg_band_apply(const mwg_level *lvl, const mwg_pairs *pairs, int npairs, int precision);
 
 /* Work distribution of the matrix-core band kernel at order 7 (kp1 = 8) for
- * MWG_PREC_FP64 and MWG_PREC_FP32.  MWG_BAND_ROWS: each wave runs all three
- * sweeps of a work unit for its own output columns (one gx, four j0), with no
- * workgroup barrier; the FP64 sweeps of the other orders always do.
+ * MWG_PREC_FP64 and MWG_PREC_FP32.  MWG_BAND_ROWS: a wave owns a share of a work
+ * unit's output.  On short levels it runs all three sweeps for four output columns
+ * (one gx, four j0) with no workgroup barrier, as the FP64 sweeps of the other
+ * orders always do; on long ones (FP64 from 131072 pairs on, FP32 from 8192 pairs
+ * or 1536 nodes on) 16 rows of every sweep, with one barrier per group.
  * MWG_BAND_TILES: the tiles of each sweep are shared out over the waves (two
  * barriers per group), the layout of the other orders' FP32 and of BF16X3.
  * MWG_BAND_AUTO (the default) is MWG_BAND_ROWS where it

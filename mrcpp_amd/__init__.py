@@ -522,9 +522,10 @@ BAND_LAYOUTS = {"auto": 0, "tiles": 1, "rows": 2}
 
 def set_band_layout(name):
     """Work distribution of the order-7 FP64/FP32 band kernel (process-wide):
-    'rows' (each wave runs all sweeps for its own output columns, no workgroup
-    barrier), 'tiles' (sweep tiles shared out over the waves, two barriers per
-    group) or 'auto' (the default: 'rows').  Results are bit-identical."""
+    'rows' (each wave owns a share of the output: all sweeps of four columns on
+    short levels, 16 rows of every sweep on long ones), 'tiles' (sweep tiles
+    shared out over the waves, two barriers per group) or 'auto' (the default:
+    'rows').  Results are bit-identical."""
     if name not in BAND_LAYOUTS:
         raise ValueError("band layout must be one of %s" % sorted(BAND_LAYOUTS))
     if lib().mwg_set_band_layout(BAND_LAYOUTS[name]) != 0:

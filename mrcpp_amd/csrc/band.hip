@@ -13,8 +13,9 @@
 //     output node are cut into work units of at most G consecutive groups
 //     (G grows with the level so the partial results fit a fixed budget), and
 //     the group codes are copied into level order.
-//  3. k_band_waves* (band_waves.h: FP64, and FP32 at order 7), k_band_mfma (the
-//     other matrix-core cases) or k_band_units (vector ALUs): persistent
+//  3. k_band_waves* (band_waves.h: FP64, and FP32 at order 7), k_band_rows (the
+//     same on long levels of order 7), k_band_mfma (the other matrix-core cases)
+//     or k_band_units (vector ALUs): persistent
 //     workgroups take units in turn or from an atomic counter; a unit
 //     accumulates its groups' 3-sweep tensor products in registers and writes
 //     one 8-block result, the node's first unit straight into the output
@@ -1022,12 +1023,12 @@ __global__ __launch_bounds__(256, N1 == 10 ? 2 : 1) void k_band_mfma(const mwg_s
 }
 
 // ---------------------------------------------------------------------------
-// 3c. order 7 (N1 = 8) on the matrix cores with wave-owned rows (FP32, long
+// 3c. order 7 (N1 = 8) on the matrix cores with wave-owned rows (FP64, FP32; long
 // levels).
 //
-// Its waves share a unit's band blocks through LDS and are five to a SIMD, which
-// on long levels beats one wave per item (k_band_waves8f, four to a SIMD, each
-// with its own operand loads); see wave_kernel for where the line lies.
+// Its waves share a unit's band blocks through LDS, which on long levels beats one
+// wave per item (k_band_waves8, k_band_waves8f, each wave with its own operand
+// loads): see wave_kernel for where the line lies.
 //
 // The same sweeps and instructions as k_band_mfma<8, PREC>, distributed so
 // that only the x -> y step crosses waves.  Wave w computes the x sweep rows
@@ -1047,6 +1048,15 @@ __global__ __launch_bounds__(256, N1 == 10 ? 2 : 1) void k_band_mfma(const mwg_s
 //   T2 (per wave) [b = 2 gx + gy][kk = i2][r = j1 + N1 (j0 - 2w)].
 // ---------------------------------------------------------------------------
 template <int PREC> struct RowGeom;
+template <> struct RowGeom<MWG_PREC_FP64> {
+    static constexpr int F = 512, T1B = 520, T1 = 2 * T1B, T2W = 512;
+    __device__ static inline int atF(int kk, int m) { return kk * 64 + (m ^ (2 * kk) ^ (16 * (kk & 1))); }
+    __device__ static inline int atT1(int gx, int kk, int j0, int i2) { return gx * T1B + kk * 64 + (((j0 + 8 * i2) ^ (2 * (i2 >> 1))) ^ (16 * (kk & 1))); }
+    __device__ static inline int atT2(int b, int kk, int r) {
+        const int gy = b & 1;
+        return b * 128 + ((kk * 16 + (r ^ (8 * gy))) ^ (16 * gy));
+    }
+};
 template <> struct RowGeom<MWG_PREC_FP32> {
     static constexpr int F = 512, T1B = 552, T1 = 2 * T1B, T2W = 576;
     __device__ static inline int atF(int kk, int m) { return kk * 64 + (m ^ (16 * (kk & 1)) ^ (4 * (kk >> 1))); }
@@ -1399,19 +1409,24 @@ template <int N1, int PREC> int mfma_grid() {
     return capped_grid(grid);
 }
 int g_band_layout = MWG_BAND_AUTO;
-// Whether a wave kernel runs: FP64 at every order, FP32 at order 7 on levels of
-// fewer than kRowsPairs pairs (the other orders' FP32 and BF16X3 sweeps keep the
-// tile-shared kernel, as order 7 does when that layout is selected).  FP32 on
-// longer levels: k_band_rows, the same bits.  Band time of an application: 16
-// Gaussians, up to some 10^4 pairs a level, rows 1.49 ms, waves 1.32; the batch of
-// 64 trees, up to some 10^5, rows 101 ms, waves 122.
-constexpr int kRowsPairs = 32768;
-bool wave_kernel(int n1, int prec, int npairs) {
-    if (prec == MWG_PREC_FP64) return n1 != 8 || g_band_layout != MWG_BAND_TILES;
-    return prec == MWG_PREC_FP32 && n1 == 8 && g_band_layout != MWG_BAND_TILES && npairs < kRowsPairs;
+// Whether a wave kernel runs: FP64 at every order, FP32 at order 7 (the other
+// orders' FP32 and BF16X3 sweeps keep the tile-shared kernel, as order 7 does when
+// that layout is selected).  Long levels of order 7 take k_band_rows, the same bits:
+// one wave per item wins by filling the card with fewer units, the row kernel by
+// fewer operand loads.  Measured level by level, waves / rows, on trees of 1 to 32
+// Gaussians and batches of 3 to 64.  FP32: 0.43-0.95 below 2000 pairs, 0.83-1.06
+// up to 8000 (1.0-1.07 where these are 1500 nodes and more), 1.0-1.1 up to 60000,
+// 1.15-1.2 at 300000.  FP64: 0.5-0.9 below 4000 pairs, 0.83-0.95 up to 30000,
+// 0.95-1.0 up to 100000, 1.02-1.04 from 150000 on and 1.03-1.06 above 250000 (boxes
+// at lower clocks 0.98 and 1.0-1.02 there).
+constexpr int kRowsPairsFp64 = 131072, kRowsPairsFp32 = 8192, kRowsNodesFp32 = 1536;
+bool wave_kernel(int n1, int prec, int npairs, int nodes) {
+    if (n1 == 8 && g_band_layout == MWG_BAND_TILES) return false;
+    if (prec == MWG_PREC_FP64) return n1 != 8 || npairs < kRowsPairsFp64;
+    return prec == MWG_PREC_FP32 && n1 == 8 && npairs < kRowsPairsFp32 && nodes < kRowsNodesFp32;
 }
-int rows_grid() {
-    static const int grid = resident_grid(k_band_rows<MWG_PREC_FP32>, 256);
+template <int PREC> int rows_grid() {
+    static const int grid = resident_grid(k_band_rows<PREC>, 256);
     return capped_grid(grid);
 }
 template <int N1, int PREC> void (*wave_kernel_of())(WaveArgs) {
@@ -1439,9 +1454,9 @@ void launch_mfma(const mwg_level *lvl, const LevelDevice &dev, const mwg_pairs *
             return;
         }
     }
-    if constexpr (PREC == MWG_PREC_FP32 && N1 == 8) {
+    if constexpr (PREC != MWG_PREC_BF16X3 && N1 == 8) {
         if (g_band_layout != MWG_BAND_TILES) {
-            hipLaunchKernelGGL((k_band_rows<PREC>), dim3(rows_grid()), dim3(256), 0, 0, dev.segs, dev.node_seg, lvl->g_off, *pr, w.grec.as<int2>(),
+            hipLaunchKernelGGL((k_band_rows<PREC>), dim3(rows_grid<PREC>()), dim3(256), 0, 0, dev.segs, dev.node_seg, lvl->g_off, *pr, w.grec.as<int2>(),
                                w.pdl.as<int4>(), w.pfo.as<long long>(), w.gstart.as<int>(), w.units.as<int4>(), w.uscan.as<long long>(), lvl->count,
                                w.partial.as<double>(), w.counter.as<int>());
             return;
@@ -1476,7 +1491,7 @@ template <int N1> struct BandL {
         if (w.codes.ensure(sizeof(unsigned) * (size_t)npairs * stride) != MWG_OK) return MWG_ERR_NOMEM;
         if (w.gstart.ensure(sizeof(int) * ((size_t)npairs + 1)) != MWG_OK) return MWG_ERR_NOMEM;
         if (w.uscan.ensure(sizeof(long long) * ((size_t)L + 1)) != MWG_OK) return MWG_ERR_NOMEM;
-        const bool waves = wave_kernel(N1, precision, npairs);
+        const bool waves = wave_kernel(N1, precision, npairs, L);
         if (w.units.ensure((waves ? sizeof(int) * kUnitInts : sizeof(int4)) * ((size_t)slots + L)) != MWG_OK) return MWG_ERR_NOMEM;
         if (w.partial.ensure(slot_bytes * (size_t)slots) != MWG_OK) return MWG_ERR_NOMEM;
         if (w.counter.ensure(sizeof(int)) != MWG_OK) return MWG_ERR_NOMEM;

@@ -1,4 +1,5 @@
-// Band sums with one wave per work item (FP64 at every order, FP32 at order 7).
+// Band sums with one wave per work item (FP64 at every order, FP32 at order 7; long
+// levels of order 7 have a kernel of their own, k_band_rows).
 //
 // A work item is a unit and one column set of its output: the x sweep's output
 // columns (gx, j0) are divided into sets of four, and a wave runs all three

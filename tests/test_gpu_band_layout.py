@@ -1,12 +1,13 @@
 """The two work distributions of the order-7 matrix-core band kernel give
 bit-identical trees.
 
-'rows' (each wave owns 16 rows of every sweep, one workgroup barrier per
-group) and 'tiles' (sweep tiles shared out over the waves) run the same
-products in the same order for every output element, so their trees must be
-equal bit for bit, in FP64 and FP32 sweeps, for Poisson and Helmholtz, for a
-single tree and for a batch.  Parity of the default layout against the
-oracle is held by the apply, batch and precision tests.
+'rows' (a wave owns a share of a unit's output: all sweeps of four columns on
+short levels, 16 rows of every sweep on long ones) and 'tiles' (sweep tiles
+shared out over the waves) run the same products in the same order for every
+output element, so their trees must be equal bit for bit, in FP64 and FP32
+sweeps, for Poisson and Helmholtz, for a single tree and for a batch, on levels
+of either side of the line between the two kernels of 'rows'.  Parity of the
+default layout against the oracle is held by the apply, batch and precision tests.
 """
 import sys
 
@@ -90,6 +91,48 @@ def test_rows_equal_tiles_batch(mr, layouts):
         assert np.array_equal(ti, ri), k
         assert np.array_equal(tc, rc), (k, float(np.abs(tc - rc).max()))
         assert np.array_equal(tn, rn), k
+
+
+@pytest.mark.parametrize("precision,trees,pairs", [("fp64", 64, 131072), ("fp32", 8, 8192)])
+def test_long_levels_equal_tiles(mr, layouts, precision, trees, pairs):
+    """A batch whose levels have so many pairs on average that the widest is past
+    the line from which 'rows' takes its kernel for long levels, while the first,
+    of eight root nodes a tree and at most eight pairs each, is before it."""
+    specs = W.batch_sources()[:trees]
+    mra = mr.MultiResolutionAnalysis((-32, 32), 7)
+    ops, inputs = {}, []
+    for b in specs:
+        f = mr.FunctionTree(mra)
+        gx = mr.GaussExp.from_sources(b["sources"])
+        mr.build_grid(f, gx)
+        mr.project(b["prec"], f, gx)
+        key = (b["mu"], b["prec"])
+        if key not in ops:
+            ops[key] = mr.PoissonOperator(mra, b["prec"]) if b["mu"] is None else mr.HelmholtzOperator(mra, b["mu"], b["prec"])
+        inputs.append((b["prec"], ops[key], f))
+    mr.set_sweep_precision(precision)
+    out = {}
+    for layout in ("tiles", "auto"):
+        mr.set_band_layout(layout)
+        outs = [mr.FunctionTree(mra) for _ in inputs]
+        stats = mr.apply_batch([(p, o, P, f) for (p, P, f), o in zip(inputs, outs)])
+        mean = sum(s["n_pairs"] for s in stats) / max(s["n_levels"] for s in stats)
+        _say("case", precision, layout, "trees", trees, "pairs a level", mean)
+        assert mean >= pairs > 64 * trees
+        out[layout] = outs
+    for k, (t, r) in enumerate(zip(out["tiles"], out["auto"])):
+        assert all(np.array_equal(x, y) for x, y in zip(t.export(), r.export())), k
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_short_levels_equal_tiles(mr, layouts, precision):
+    """A tree with fewer pairs in all than either line."""
+    src = W.random_sources(3, 1, 1.0)
+    (ti, tc, tn), tst = _apply(mr, src, 7, 16, 1e-4, None, "tiles", precision)
+    (ri, rc, rn), rst = _apply(mr, src, 7, 16, 1e-4, None, "auto", precision)
+    _say("case", precision, "pairs", rst["n_pairs"], "nodes", rst["level_nodes"])
+    assert rst["n_pairs"] < 8192 and max(rst["level_nodes"]) < 1536
+    assert np.array_equal(ti, ri) and np.array_equal(tc, rc) and np.array_equal(tn, rn)
 
 
 def test_unit_groups_change_only_the_last_bits(mr, layouts):
