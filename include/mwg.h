@@ -461,7 +461,10 @@ mwg_status mwg_operator_nodes(int kp1, const double *left, const double *right, 
  * generated node, its scaling block at -in_off - 1 (wavelet blocks zero).
  * scale[k] is the node's scale, out_off[k] its offset in out; norms[9 k] the 8
  * component norms and the square norm.  Sums take no fused multiply-add: the
- * host's order of operations. */
+ * host's order of operations.  Products sum in another order: a node differs from
+ * the host's by at most 36 2^-53 |f| |g| / sqrt(volume) of two operands' norms in
+ * it, which is far more than the last bits of a product of factors that hardly
+ * overlap (the host's own rounding there is as large). */
 #define MWG_MAX_OPERANDS 8
 typedef struct {
     int kp1;
