@@ -59,7 +59,8 @@ mwg_status mwg_download_many(int n, void *const *dst, const void *const *src, co
 /* Streams `bytes` of device memory to sink(ctx, piece, offset, size), in order
  * and on the calling thread: pieces of `piece_bytes` (0 < piece_bytes <= 4 MiB,
  * the last may be shorter) land in page-locked memory, and while sink takes one
- * the next are on their way.  A piece is valid during its call only. */
+ * the next are on their way.  A piece is valid during its call only; sink must
+ * not call into the library (downloads share the memory). */
 typedef void (*mwg_sink)(void *ctx, const void *piece, size_t offset, size_t size);
 mwg_status mwg_download_stream(const void *src, size_t bytes, size_t piece_bytes, mwg_sink sink, void *ctx);
 /* Upload through a pinned staging ring and return without waiting: src may be

@@ -13,13 +13,13 @@
 namespace mrcpp {
 namespace device {
 
-void download_rows(const double *src, size_t row_doubles, const std::vector<double *> &dst) {
+void stream_rows(const double *src, size_t row_doubles, size_t rows, const std::function<void(size_t, const double *)> &take, int threads) {
     struct Job {
-        const std::vector<double *> &dst;
+        const std::function<void(size_t, const double *)> &take;
         size_t row; // bytes
         int threads;
-    } job{dst, sizeof(double) * row_doubles, std::max(1, omp_get_max_threads() - 2)}; // two cores left to the runtime's threads
-    const size_t bytes = dst.size() * job.row;
+    } job{take, sizeof(double) * row_doubles, threads};
+    const size_t bytes = rows * job.row;
     // whole rows per piece, four pieces or more where the rows fill them (the
     // host then works on one while the link carries the next)
     const size_t target = std::min<size_t>(std::max<size_t>(bytes / 4, size_t(512) << 10), size_t(4) << 20);
@@ -30,12 +30,17 @@ void download_rows(const double *src, size_t row_doubles, const std::vector<doub
         // a thread's share is at least 64 KiB: waking one costs about as much
         const int threads = std::min<long>(j.threads, std::max<long>(1, (long)(size >> 16)));
 #pragma omp parallel for schedule(static) num_threads(threads) if (threads > 1)
-        for (long i = 0; i < n; i++)
-            if (double *d = j.dst[first + i]) std::memcpy(d, static_cast<const char *>(piece) + i * j.row, j.row);
+        for (long i = 0; i < n; i++) j.take(first + i, reinterpret_cast<const double *>(static_cast<const char *>(piece) + i * j.row));
     };
     check(mwg_download_stream(src, bytes, piece, place, &job), "download");
 }
 
+void download_rows(const double *src, size_t row_doubles, const std::vector<double *> &dst) {
+    const auto place = [&](size_t i, const double *row) {
+        if (dst[i]) std::memcpy(dst[i], row, sizeof(double) * row_doubles);
+    };
+    stream_rows(src, row_doubles, dst.size(), place, std::max(1, omp_get_max_threads() - 2)); // two cores left to the runtime's threads
+}
 
 void check(mwg_status s, const char *what) {
     if (s != MWG_OK) throw Error(std::string(what) + ": " + mwg_last_error());

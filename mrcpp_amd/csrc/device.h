@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
+#include <functional>
 #include <mutex>
 #include <string>
 #include <unordered_map>
@@ -79,8 +80,10 @@ private:
 };
 
 // Rows of device memory (row i: row_doubles at src + i row_doubles) to
-// dst[i] each (null: skipped), the host threads placing one piece while the
-// next are on the link.
+// take(i, row) each, by up to `threads` host threads while the next rows are on the
+// link; take must not throw nor call into the device layer.
+void stream_rows(const double *src, size_t row_doubles, size_t rows, const std::function<void(size_t, const double *)> &take, int threads);
+// The same to dst[i] each (null: skipped), by all host threads.
 void download_rows(const double *src, size_t row_doubles, const std::vector<double *> &dst);
 
 // Page-locked host buffer, grown on demand (contents are not kept).

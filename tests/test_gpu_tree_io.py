@@ -88,3 +88,31 @@ def test_text_file_of_apply_matches_the_oracle(mr, orc, tmp_path):
     assert pb == ob
     assert pv.shape == ov.shape
     assert np.abs(pv - ov).max() <= 1e-12 * np.abs(ov).max()
+
+
+@pytest.mark.parametrize("order,prec,gaussians", [(3, 1e-3, 1), (7, 1e-5, 4)])
+def test_resident_tree_saves_the_file_of_its_host_copy(mr, tmp_path, order, prec, gaussians):
+    """A tree in HBM is written node by node as it arrives (an export before
+    leaves it there); once evalf has made the host copy the file is written from
+    that: the same bytes, and the same tree when read back.  One piece of the
+    download, and several."""
+    mra = mr.MultiResolutionAnalysis((-16, 16), order)
+    gx = mr.GaussExp.from_sources(W.random_sources(8, gaussians, 3.0))
+    f = mr.FunctionTree(mra)
+    mr.build_grid(f, gx)
+    mr.project(prec, f, gx)
+    g = mr.FunctionTree(mra)
+    mr.apply(prec, g, mr.PoissonOperator(mra, prec), f)
+    ref = g.export()
+    g.saveTree(str(tmp_path / "resident"))
+    g.evalf((0.1, 0.2, 0.3))
+    g.saveTree(str(tmp_path / "host"))
+    print("case", order, "nodes", len(ref[0]), "bytes", (tmp_path / "host.tree").stat().st_size)
+    assert (tmp_path / "resident.tree").read_bytes() == (tmp_path / "host.tree").read_bytes()
+    b = mr.FunctionTree(mra)
+    b.loadTree(str(tmp_path / "resident"))
+    assert all(np.array_equal(x, y) for x, y in zip(ref, b.export()))
+    h = mr.FunctionTree(mra)
+    mr.apply(prec, h, mr.PoissonOperator(mra, prec), f)
+    with pytest.raises(mr.MRCPPError):
+        h.saveTree(str(tmp_path / "missing" / "h"))
