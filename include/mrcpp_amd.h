@@ -126,8 +126,8 @@ int mrcpp_operator_node(void *oper, int term, int depth, int l, int comp, double
 int mrcpp_kernel_terms(int kind, double mu, double eps, double r_min, double r_max, double *alpha, double *coef, int cap);
 
 /* Sweep precision of later mrcpp_apply calls on this thread: 0 FP64 (default,
- * matrix cores), 1 FP32, 2 BF16x3, 3 FP64 on the vector ALUs.  No reference
- * counterpart (the reference computes in FP64 only). */
+ * matrix cores), 1 FP32 (the faster form at order 7 only), 2 BF16x3, 3 FP64 on the
+ * vector ALUs.  No reference counterpart (the reference computes in FP64 only). */
 int mrcpp_set_sweep_precision(int precision);
 int mrcpp_get_sweep_precision(void);
 /* Whether later mrcpp_apply calls on this thread form each breadth-first

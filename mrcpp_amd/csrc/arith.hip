@@ -20,9 +20,10 @@ namespace {
 
 // coefs_o = 0; coefs_o += c_i coefs_i, operand by operand, and the norms (the
 // order of block_norms).  Bound by the reads' latency: every load of a thread's
-// values is in flight at once and nothing goes through LDS, so eight workgroups
-// share a CU (one kernel for sums and products held two; 273 order-7 nodes a
-// launch: 46 -> 13 us).
+// values is in flight at once, and as nothing goes through LDS the registers set
+// how many workgroups share a CU, eight at orders 3 and 5, five at order 7, two at
+// order 9 (one kernel for sums and products held two; 273 order-7 nodes a launch:
+// 46 -> 13 us).
 template <int N1>
 __global__ __launch_bounds__(kThreads) void k_sum(mwg_combine cb, const long long *in_off, const long long *out_off, double *out, double *norms) {
     constexpr int N3 = N1 * N1 * N1, PT = (8 * N3 + kThreads - 1) / kThreads;
@@ -65,8 +66,8 @@ __global__ __launch_bounds__(kThreads) void k_sum(mwg_combine cb, const long lon
 
 // Products.  Each pass takes its direction's filters and its map between
 // coefficients and values, so an operand takes three passes and the way back
-// three (before, six each on the vector units: 114 -> 46 us a launch at order 9,
-// 36 -> 18 at order 5), and the values are multiplied in the registers the
+// three (before, six each on the vector units: 162 -> 46 us a launch at order 9,
+// 43 -> 18 at order 5), and the values are multiplied in the registers the
 // third pass leaves them in.  Bound by the chain of loads, passes and barriers of a node.
 template <int N1>
 __global__ __launch_bounds__(MwShape<N1>::THREADS, MwShape<N1>::OCC) void k_product(mwg_combine cb, const long long *in_off, const int *scale, const long long *out_off,

@@ -27,10 +27,12 @@
 // [Oy columns] and the z sweep as [Oz^T rows] x [T2 columns].  x -> y needs one
 // transposition, through LDS private to the wave.
 //
-// Every output element goes through the same products in the same order as in
-// k_band_mfma (f64 and f32 products on the matrix cores are one fused
-// multiply-add per contracted index, in index order, whichever instruction
-// shape forms them), so order 7 gives the same bits with either.
+// Every output element goes through the same products as in k_band_mfma, at order
+// 7 in the same order (f64 and f32 products on the matrix cores are one fused
+// multiply-add per contracted index, in index order, whichever instruction shape
+// forms them), so order 7 gives the same bits with either.  At orders 3, 5 and 9
+// the z product of a group that does not fill its mask is formed from zero and
+// then added.
 //
 // Results: a node's first unit is written to the node itself, each further unit
 // to a slot in the order of WaveMap, which each wave writes in whole 512-byte
@@ -218,12 +220,13 @@ __device__ inline double mma4(double a, double b, double c) { return __builtin_a
 // ---------------------------------------------------------------------------
 // Order 7, FP64.  Item = (unit, gx, j0 / 4), a workgroup's four waves taking
 // the four items of a unit (they read the same operands at about the same time,
-// through one L1): a group without gx in its mask is passed over.  x: 64 lines x 4 columns, eight 4x4x4 products from the band
-// block held in registers; y: per gy, j0 pair and i2 tile, 4x4x4 products whose
+// through one L1): a group without gx in its mask is passed over.  x: 64 lines x 4
+// columns, eight 4x4x4 products from the band block held in registers; y: per gy,
+// j0 pair and i2 tile, 4x4x4 products whose
 // result lanes are (j0', j1) x i2 quarter; z: 16x16x4 into [j0 pair][gy].
 // T1[j0][i2][i1] in LDS at 84 j0 + 10 i2 + 2 (i1 & 3) + (i1 >> 2): both k
-// steps of an operand in one 16-byte read, writes and reads without bank
-// conflicts.
+// steps of an operand in one 16-byte read.  The counters still put half of the LDS
+// cycles down to bank conflicts (a third at FP32); the loop does not wait for them.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256, 4) void k_band_waves8(WaveArgs a) {
     constexpr int SJ = 84, SI = 10;

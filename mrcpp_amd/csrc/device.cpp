@@ -13,9 +13,11 @@
 namespace mrcpp {
 namespace device {
 
-void stream_rows(const double *src, size_t row_doubles, size_t rows, const std::function<void(size_t, const double *)> &take, int threads) {
+namespace {
+
+template <class Take> void stream(const double *src, size_t row_doubles, size_t rows, const Take &take, int threads) {
     struct Job {
-        const std::function<void(size_t, const double *)> &take;
+        const Take &take;
         size_t row; // bytes
         int threads;
     } job{take, sizeof(double) * row_doubles, threads};
@@ -35,11 +37,17 @@ void stream_rows(const double *src, size_t row_doubles, size_t rows, const std::
     check(mwg_download_stream(src, bytes, piece, place, &job), "download");
 }
 
+} // namespace
+
+void stream_rows(const double *src, size_t row_doubles, size_t rows, const std::function<void(size_t, const double *)> &take, int threads) {
+    stream(src, row_doubles, rows, take, threads);
+}
+
 void download_rows(const double *src, size_t row_doubles, const std::vector<double *> &dst) {
     const auto place = [&](size_t i, const double *row) {
         if (dst[i]) std::memcpy(dst[i], row, sizeof(double) * row_doubles);
     };
-    stream_rows(src, row_doubles, dst.size(), place, std::max(1, omp_get_max_threads() - 2)); // two cores left to the runtime's threads
+    stream(src, row_doubles, dst.size(), place, std::max(1, omp_get_max_threads() - 2)); // two cores left to the runtime's threads
 }
 
 void check(mwg_status s, const char *what) {

@@ -6,7 +6,8 @@ tests/test_arith_oracle.py pins to closed forms.
 Inputs are projected on the host so both sides start from bit-identical trees.
 Bar: identical node sets; coefficients within 1e-14 relative L2 of the
 oracle's (sums without fused multiply-adds in the same order; the device's
-products, norm sums and bottom-up transform round differently).
+products, norm sums and bottom-up transform round differently; factors that hardly
+overlap have a bar of their own in tests/test_gpu_arith_sizes.py).
 """
 import math
 import sys
