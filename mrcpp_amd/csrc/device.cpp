@@ -16,6 +16,8 @@ namespace device {
 namespace {
 
 template <class Take> void stream(const double *src, size_t row_doubles, size_t rows, const Take &take, int threads) {
+    // the pieces land in memory that every download shares
+    std::lock_guard<std::recursive_mutex> lock(api_mutex());
     struct Job {
         const Take &take;
         size_t row; // bytes

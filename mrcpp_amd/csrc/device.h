@@ -23,7 +23,8 @@ void ensure_init();
 // Process-wide lock of the device path.  The device layer keeps its scratch
 // buffers, staging ring and stream per process, so calls that use it run one
 // at a time: every mrcpp_* C ABI entry point and apply_batch() hold this
-// (recursive) lock for their whole call.
+// (recursive) lock for their whole call, the handing over of a tree's coefficients
+// while they stream.
 std::recursive_mutex &api_mutex();
 // whether a GPU is present and the device layer initialised
 bool available();

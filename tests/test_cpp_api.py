@@ -43,3 +43,14 @@ def test_cpp_api_program_on_gpu():
     assert r.returncode == 0, r.stdout + r.stderr
     assert "PASSED: 0 failed checks" in r.stdout
     assert "FAIL " not in r.stdout
+
+
+@pytest.mark.gpu
+def test_two_threads_bring_their_trees_out_of_hbm(tmp_path):
+    """evalf and saveTree of trees in HBM from two host threads at once: the
+    downloads share page-locked memory, so they have to take turns."""
+    exe = os.path.join(os.path.dirname(EXE), "two_threads")
+    r = subprocess.run([exe, str(tmp_path)], capture_output=True, text=True, timeout=100)
+    print(r.stdout, flush=True)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert "PASSED: 0 wrong" in r.stdout
