@@ -226,7 +226,8 @@ __device__ inline double mma4(double a, double b, double c) { return __builtin_a
 // result lanes are (j0', j1) x i2 quarter; z: 16x16x4 into [j0 pair][gy].
 // T1[j0][i2][i1] in LDS at 84 j0 + 10 i2 + 2 (i1 & 3) + (i1 >> 2): both k
 // steps of an operand in one 16-byte read.  The counters still put half of the LDS
-// cycles down to bank conflicts (a third at FP32); the loop does not wait for them.
+// cycles down to bank conflicts (a third at FP32), while the waves wait 0.13 of theirs
+// for anything.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256, 4) void k_band_waves8(WaveArgs a) {
     constexpr int SJ = 84, SI = 10;
